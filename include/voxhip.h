@@ -291,6 +291,17 @@ int vx_mc_emit(const float* u, int nx, int ny, int nz, float iso, const int8_t* 
                const int8_t* edges, const int64_t* vincl, const int64_t* tincl,
                const double* bounds, double* verts, int64_t* faces, void* stream);
 
+/* Marching cubes of the whole field in two calls: vx_mc_classify fills the workspace `ws`
+ * (vx_mc_workspace_bytes, 8-byte aligned; -1: sizes out of range) and totals = {vertices,
+ * triangles} (device); vx_mc_write, with those totals, the mesh vx_mc_emit writes (same
+ * vertices, triangles and order).  u, iso and ws must be the classify call's. */
+int64_t vx_mc_workspace_bytes(int nx, int ny, int nz);
+int vx_mc_classify(const float* u, int nx, int ny, int nz, float iso, const int8_t* count,
+                   void* ws, int64_t* totals, void* stream);
+int vx_mc_write(const float* u, int nx, int ny, int nz, float iso, const int8_t* count,
+                const int8_t* edges, void* ws, int64_t n_verts, int64_t n_faces,
+                const double* bounds, double* verts, int64_t* faces, void* stream);
+
 /* Zero n elements (a fill kernel, safe inside captured graphs). */
 int vx_zero(int dtype, void* p, int64_t n, void* stream);
 

@@ -4,10 +4,11 @@
 // the host and calls PyMCubes on the CPU.
 //
 // Here the field stays on the device: vx_extract_fields evaluates the trilinear SDF at
-// the lattice points (torch.linspace's arithmetic), and marching cubes runs as two
-// passes over lattice points with a scan between them: count (crossing edges owned by
-// each point, triangles of the cube at each point), then emit (vertices on the owned
-// edges, triangles by table).  Every vertex sits on exactly one lattice edge and is
+// the lattice points (torch.linspace's arithmetic), and marching cubes counts (crossing
+// edges owned by each point, triangles of the cube at each point), scans and writes
+// (vertices on the owned edges, triangles by table): vx_mc_classify / vx_mc_write on
+// bit rows of the lattice, vx_mc_count / vx_mc_emit with per-point counts and a scan of the
+// caller's between them.  Every vertex sits on exactly one lattice edge and is
 // shared by all triangles that use that edge, so the mesh is indexed without a hash.
 //
 // The triangle table is generated here (vx_mc_tables), not transcribed: for each of the
@@ -188,8 +189,80 @@ struct FieldArgs {
   float* u;             // [n0, n1, n2]
 };
 
-// One thread per lattice point; 3-D grid (z chunks of 256, y, x).
+// One axis of the lattice: the cell and the weights of its points, as the drop-in
+// grid_sample's Tri::init has them, with the in-grid bits of the cell's two lattice lines.
+struct FieldAxis {
+  int off0, off1;    // element offsets of the two (clamped) lattice lines
+  float w0, w1;
+  int x0;            // cell (unclamped)
+  unsigned in;
+};
+
+__device__ __forceinline__ FieldAxis field_axis(const FieldArgs& a, int ax, int i, int size,
+                                                int64_t stride) {
+#pragma clang fp contract(off)
+  const float p = linspace_at(a.bmin[ax], a.bmax[ax], a.n[ax], i);
+  const float f = world_to_index(p, a.mn[ax], a.mx[ax] - a.mn[ax], size);
+  const float ff = floorf(f);
+  FieldAxis r;
+  r.x0 = sat_f2i(ff);
+  r.w0 = (ff + 1.f) - f;
+  r.w1 = f - ff;
+  r.off0 = (int)(clamp_index(r.x0, size) * stride);
+  r.off1 = (int)(clamp_index(r.x0 + 1, size) * stride);
+  r.in = ((unsigned)r.x0 < (unsigned)size ? 1u : 0u) |
+         ((unsigned)(r.x0 + 1) < (unsigned)size ? 2u : 0u);
+  return r;
+}
+
+// The lattice field, a thread's z of kFieldRows consecutive rows (3-D grid: z chunks of 256,
+// row groups, x).  Bound by instruction issue: with one point per thread the three axes'
+// divisions and 64-bit addresses of every point took 735 us for a 512^3 lattice of a 256^3
+// grid (537 MB written).  Here the x axis is made once per thread, the z axis once per
+// thread, the y axis once per row in the lanes of the block that hold it (LDS), and a
+// row whose cell is the previous row's keeps its eight corner values (the lattice is
+// finer than the grid).  Each point's value is the drop-in grid_sample's, bit for bit.
+constexpr int kFieldRows = 8;
 __global__ void __launch_bounds__(256) k_extract_fields(FieldArgs a) {
+#pragma clang fp contract(off)
+  __shared__ FieldAxis ys[kFieldRows];
+  const int k = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.z;
+  const int j0 = blockIdx.y * kFieldRows;
+  const int rows = min(kFieldRows, a.n[1] - j0);
+  if ((int)threadIdx.x < rows)
+    ys[threadIdx.x] = field_axis(a, 1, j0 + threadIdx.x, a.g.Y, a.g.sy);
+  const FieldAxis x = field_axis(a, 0, i, a.g.X, a.g.sx);
+  const FieldAxis z = field_axis(a, 2, min(k, a.n[2] - 1), a.g.Z, a.g.sz);
+  __syncthreads();
+  if (k >= a.n[2]) return;
+  float* out = a.u + ((int64_t)i * a.n[1] + j0) * a.n[2] + k;
+  float v[8];
+  int cell = 0;
+  for (int r = 0; r < rows; ++r) {
+    const FieldAxis y = ys[r];
+    const int yc = __builtin_amdgcn_readfirstlane(y.x0);
+    if (r == 0 || yc != cell) {
+      cell = yc;
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        v[c] = a.sdf[(c >> 2 ? x.off1 : x.off0) + (c >> 1 & 1 ? y.off1 : y.off0) +
+                     (c & 1 ? z.off1 : z.off0)];
+    }
+    float acc = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int bx = c >> 2, by = c >> 1 & 1, bz = c & 1;
+      const float w = ((bz ? z.w1 : z.w0) * (by ? y.w1 : y.w0)) * (bx ? x.w1 : x.w0);
+      const float t = acc + v[c] * w;
+      acc = (x.in >> bx & y.in >> by & z.in >> bz & 1u) ? t : acc;
+    }
+    out[(int64_t)r * a.n[2]] = a.scale * acc;
+  }
+}
+
+// The same, one point per thread (3-D grid: z chunks of 256, y, x), for grids whose element
+// offsets pass 32 bits.
+__global__ void __launch_bounds__(256) k_extract_fields_wide(FieldArgs a) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, i = blockIdx.z;
   if (k >= a.n[2]) return;
   const float px = linspace_at(a.bmin[0], a.bmax[0], a.n[0], i);
@@ -204,7 +277,7 @@ __global__ void __launch_bounds__(256) k_extract_fields(FieldArgs a) {
   a.u[((int64_t)i * a.n[1] + j) * a.n[2] + k] = a.scale * v;
 }
 
-// ---- marching cubes ---------------------------------------------------------------------
+// ---- marching cubes, per-point counts ------------------------------------------------------
 
 struct McArgs {
   const float* u;
@@ -295,6 +368,341 @@ __global__ void __launch_bounds__(256) k_mc_emit(McArgs a, const int64_t* __rest
   }
 }
 
+// ---- marching cubes on bit rows ----------------------------------------------------------
+// The passes above keep two int64 per lattice point and scan them: 2 GiB written, and read
+// and written three times more, for a 512^3 lattice of which one point in a hundred touches
+// the surface (5.1 ms).  Here a point's side of the threshold is one bit: 64 consecutive
+// points of a z row make a 64-bit word (a row's last word is padded), and every later
+// question is asked of words -- which of a group's edges cross, which of its cubes are cut,
+// how many vertices come before a point.  Three passes:
+//   k_mc_below   the field once, 64 points per ballot (bound by the read);
+//   k_mc_groups  per group (word) the vertices its points own and the triangles of its
+//                cubes, with their prefix over the block's groups (bits from L2);
+//   k_mc_write   the groups that hold any, a lane per point: a vertex number is the
+//                group's offset plus the popcounts below the point's bit.
+// Vertices and triangles come in the order of the passes above: by point, then by axis or
+// by the table.
+constexpr int kMcThreads = 256;
+
+struct McGroups {
+  int64_t words;      // words of a z row
+  int64_t total;      // groups: nx * ny * words
+  uint64_t* bits;     // [total] u < iso
+  uint64_t* pre;      // [total] vertices | triangles << 32 of the block's earlier groups
+  int64_t* blk;       // [2 * blocks] per block: vertices, triangles (then their offsets)
+};
+
+// Row of group q (32-bit division where the groups' numbers fit: the 64-bit one is a long
+// sequence).
+__device__ __forceinline__ int64_t mc_row(const McGroups& g, int64_t q) {
+  if (g.total <= 0x7fffffff) return (int64_t)((uint32_t)q / (uint32_t)g.words);
+  return q / g.words;
+}
+
+__global__ void __launch_bounds__(256) k_mc_below(const float* __restrict__ u, int nz, float iso,
+                                                  McGroups g) {
+  constexpr int U = 8;  // words per wave and round: their loads are all in flight together
+  const int lane = threadIdx.x & 63;
+  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int64_t q0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + wave) * U;
+  for (; q0 < g.total; q0 += waves * U) {
+    float v[U];
+    bool in[U];
+    int64_t row = mc_row(g, q0);
+    int w = (int)(q0 - row * g.words);
+#pragma unroll
+    for (int e = 0; e < U; ++e) {
+      const int z = 64 * w + lane;
+      in[e] = q0 + e < g.total && z < nz;
+      v[e] = in[e] ? u[row * nz + z] : 0.f;
+      if (++w == g.words) {
+        w = 0;
+        ++row;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < U; ++e) {
+      const uint64_t b = __ballot(in[e] && v[e] < iso);
+      if (lane == 0 && q0 + e < g.total) g.bits[q0 + e] = b;
+    }
+  }
+}
+
+// The words of a group's neighbourhood: b[di][dj] the word at (i + di, j + dj, w), n[di][dj]
+// the row's next word (0 past the row), as far as they lie in the lattice (else 0).
+template <int D>
+struct McWords {
+  uint64_t b[D][D], n[D][D];
+  int nzw;         // points of this word (64, or fewer in a row's last)
+  bool ix, jy;     // i + 1, j + 1 in the lattice
+  bool more;       // the row goes on past this word
+};
+
+template <int D>
+__device__ __forceinline__ void mc_words(const McArgs& a, const McGroups& g, int i, int j, int w,
+                                         McWords<D>& m) {
+  m.nzw = min(64, a.nz - 64 * w);
+  m.ix = i + 1 < a.nx;
+  m.jy = j + 1 < a.ny;
+  m.more = w + 1 < g.words;
+#pragma unroll
+  for (int di = 0; di < D; ++di)
+#pragma unroll
+    for (int dj = 0; dj < D; ++dj) {
+      const bool in = i + di < a.nx && j + dj < a.ny;
+      const int64_t q = ((int64_t)min(i + di, a.nx - 1) * a.ny + min(j + dj, a.ny - 1)) * g.words + w;
+      m.b[di][dj] = in ? g.bits[q] : 0;
+      m.n[di][dj] = in && m.more ? g.bits[q + 1] : 0;
+    }
+}
+
+__device__ __forceinline__ uint64_t low_bits(int n) { return n >= 64 ? ~0ull : (1ull << n) - 1; }
+
+// Word of the points one further along z, and the bits of the word's points that have one.
+__device__ __forceinline__ uint64_t mc_up(uint64_t b, uint64_t next) { return b >> 1 | next << 63; }
+template <int D>
+__device__ __forceinline__ uint64_t mc_zmask(const McWords<D>& m) {
+  return low_bits(m.more ? 64 : m.nzw - 1);
+}
+
+// Crossing edges along x, y and z owned by the points of the word at (di, dj).
+template <int D>
+__device__ __forceinline__ void mc_edges(const McArgs& a, const McWords<D>& m, int i, int j, int di,
+                                         int dj, uint64_t e[3]) {
+  const uint64_t b = m.b[di][dj], in = low_bits(m.nzw);
+  e[0] = i + di + 1 < a.nx ? (b ^ m.b[di + 1][dj]) & in : 0;
+  e[1] = j + dj + 1 < a.ny ? (b ^ m.b[di][dj + 1]) & in : 0;
+  e[2] = (b ^ mc_up(b, m.n[di][dj])) & mc_zmask(m);
+}
+
+// Configuration words of the word's cubes (bit k of word c: corner c of cube k is below) and
+// the cubes that are cut.
+template <int D>
+__device__ __forceinline__ uint64_t mc_cubes(const McWords<D>& m, uint64_t c[8]) {
+  uint64_t all = ~0ull, any = 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const uint64_t b = m.b[q & 1][q >> 1 & 1];
+    c[q] = q >> 2 ? mc_up(b, m.n[q & 1][q >> 1 & 1]) : b;
+    all &= c[q];
+    any |= c[q];
+  }
+  return m.ix && m.jy ? any & ~all & mc_zmask(m) : 0;
+}
+
+__device__ __forceinline__ int mc_config(const uint64_t c[8], int k) {
+  int cfg = 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) cfg |= (int)(c[q] >> k & 1) << q;
+  return cfg;
+}
+
+__global__ void __launch_bounds__(kMcThreads) k_mc_groups(McArgs a, McGroups g) {
+  __shared__ int8_t count[256];
+  __shared__ uint64_t wave_sum[kMcThreads / 64];
+  count[threadIdx.x] = a.count[threadIdx.x];
+  __syncthreads();
+  const int64_t q = (int64_t)blockIdx.x * kMcThreads + threadIdx.x;
+  uint32_t nv = 0, nt = 0;
+  if (q < g.total) {
+    const int64_t row = mc_row(g, q);
+    const int w = (int)(q - row * g.words), i = (int)(row / a.ny), j = (int)(row - (int64_t)i * a.ny);
+    McWords<2> m;
+    mc_words(a, g, i, j, w, m);
+    uint64_t e[3], c[8];
+    mc_edges(a, m, i, j, 0, 0, e);
+    nv = (uint32_t)(__popcll(e[0]) + __popcll(e[1]) + __popcll(e[2]));
+    for (uint64_t cut = mc_cubes(m, c); cut; cut &= cut - 1)
+      nt += count[mc_config(c, __ffsll((unsigned long long)cut) - 1)];
+  }
+  // block-wide exclusive prefix of both counts (at most 256 * 192 and 256 * 320)
+  const uint64_t own = (uint64_t)nt << 32 | nv;
+  const uint64_t inc = (uint64_t)wave_incl_scan_i64((int64_t)own);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 63) wave_sum[wave] = inc;
+  __syncthreads();
+  uint64_t before = 0, total = 0;
+#pragma unroll
+  for (int k = 0; k < kMcThreads / 64; ++k) {
+    if (k < wave) before += wave_sum[k];
+    total += wave_sum[k];
+  }
+  if (q < g.total) g.pre[q] = before + inc - own;
+  if (threadIdx.x == 0) {
+    g.blk[2 * blockIdx.x] = (int64_t)(total & 0xffffffffull);
+    g.blk[2 * blockIdx.x + 1] = (int64_t)(total >> 32);
+  }
+}
+
+// Exclusive scan of the blocks' counts in place by one workgroup, eight blocks per thread
+// and round; totals[0] and [1] receive the numbers of vertices and triangles.
+__global__ void __launch_bounds__(1024) k_mc_scan(int64_t* __restrict__ blk, int64_t blocks,
+                                                  int64_t* __restrict__ totals) {
+  constexpr int U = 8;
+  __shared__ int64_t lds[2][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int64_t carry[2] = {0, 0};
+  for (int64_t base = 0; base < blocks; base += 1024 * U) {
+    const int64_t b0 = base + (int64_t)threadIdx.x * U;
+    int64_t v[U][2], s[2] = {0, 0}, inc[2];
+#pragma unroll
+    for (int e = 0; e < U; ++e)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        v[e][c] = b0 + e < blocks ? blk[2 * (b0 + e) + c] : 0;
+        s[c] += v[e][c];
+      }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      inc[c] = wave_incl_scan_i64(s[c]);
+      if (lane == 63) lds[c][wave] = inc[c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      int64_t off = carry[c] + inc[c] - s[c];
+      for (int k = 0; k < 16; ++k) {
+        if (k < wave) off += lds[c][k];
+        carry[c] += lds[c][k];
+      }
+#pragma unroll
+      for (int e = 0; e < U; ++e) {
+        if (b0 + e < blocks) blk[2 * (b0 + e) + c] = off;
+        off += v[e][c];
+      }
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    totals[0] = carry[0];
+    totals[1] = carry[1];
+  }
+}
+
+struct McWorld {
+  int on;
+  double bmin[3], ext[3];
+};
+
+// A wave takes 64 consecutive groups and works through those that hold a vertex or a
+// triangle, a lane per point of the group.
+__global__ void __launch_bounds__(kMcThreads) k_mc_write(McArgs a, McGroups g, McWorld wd,
+                                                         int64_t nv, int64_t nt,
+                                                         double* __restrict__ verts,
+                                                         int64_t* __restrict__ faces) {
+  const int lane = threadIdx.x & 63;
+  const int64_t q0 = (int64_t)blockIdx.x * kMcThreads + (threadIdx.x & ~63);
+  const int64_t q = q0 + lane;
+  // the group's counts: the next group's prefix less its own (the block's first group of the
+  // next block starts from that block's offsets)
+  bool holds = false;
+  if (q < g.total) {
+    const int64_t vo = g.blk[2 * blockIdx.x], to = g.blk[2 * blockIdx.x + 1];
+    const bool last = threadIdx.x == kMcThreads - 1 || q + 1 == g.total;
+    const uint64_t here = g.pre[q];
+    uint64_t next;
+    if (!last) {
+      next = g.pre[q + 1];
+    } else {
+      const bool end = blockIdx.x + 1 == gridDim.x;
+      const int64_t v1 = end ? nv : g.blk[2 * (blockIdx.x + 1)];
+      const int64_t t1 = end ? nt : g.blk[2 * (blockIdx.x + 1) + 1];
+      next = (uint64_t)(t1 - to) << 32 | (uint64_t)(v1 - vo);
+    }
+    holds = next != here;
+  }
+  const int64_t sx = (int64_t)a.ny * a.nz, sy = a.nz;
+  const int nn[3] = {a.nx, a.ny, a.nz};
+  for (uint64_t todo = __ballot(holds); todo; todo &= todo - 1) {
+    const int64_t qq = q0 + (__ffsll((unsigned long long)todo) - 1);
+    const int64_t row = mc_row(g, qq);
+    const int w = (int)(qq - row * g.words), i = (int)(row / a.ny), j = (int)(row - (int64_t)i * a.ny);
+    const int k = 64 * w + lane;
+    McWords<3> m;
+    mc_words(a, g, i, j, w, m);
+    // first vertex number of the groups at (i + di, j + dj, w) and of their rows' next ones
+    int64_t v0[2][2], v1[2][2];
+    uint64_t ed[2][2][3];
+#pragma unroll
+    for (int di = 0; di < 2; ++di)
+#pragma unroll
+      for (int dj = 0; dj < 2; ++dj) {
+        const bool in = i + di < a.nx && j + dj < a.ny;
+        const int64_t qn = in ? ((int64_t)(i + di) * a.ny + (j + dj)) * g.words + w : qq;
+        v0[di][dj] = g.blk[2 * (qn / kMcThreads)] + (int64_t)(g.pre[qn] & 0xffffffffull);
+        const int64_t qm = in && m.more ? qn + 1 : qn;
+        v1[di][dj] = g.blk[2 * (qm / kMcThreads)] + (int64_t)(g.pre[qm] & 0xffffffffull);
+        mc_edges(a, m, i, j, di, dj, ed[di][dj]);
+      }
+    const uint64_t lt = low_bits(lane);
+    if ((ed[0][0][0] | ed[0][0][1] | ed[0][0][2]) >> lane & 1) {
+      const int64_t p = (i * sx + j * sy) + k;
+      const int64_t step[3] = {sx, sy, 1};
+      int64_t vid = v0[0][0] + __popcll(ed[0][0][0] & lt) + __popcll(ed[0][0][1] & lt) +
+                    __popcll(ed[0][0][2] & lt);
+      const double f1 = a.u[p];
+#pragma unroll
+      for (int ax = 0; ax < 3; ++ax) {
+        if (!(ed[0][0][ax] >> lane & 1)) continue;
+        const double f2 = a.u[p + step[ax]];
+        double v[3] = {(double)i, (double)j, (double)k};
+        v[ax] += ((double)a.iso - f1) / (f2 - f1);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          double o = v[c];
+          if (wd.on) o = o / (double)(nn[c] - 1) * wd.ext[c] + wd.bmin[c];
+          verts[3 * vid + c] = o;
+        }
+        ++vid;
+      }
+    }
+    uint64_t c[8];
+    const uint64_t cut = mc_cubes(m, c);
+    const bool mine = cut >> lane & 1;
+    const int cfg = mine ? mc_config(c, lane) : 0;
+    const int n = mine ? a.count[cfg] : 0;
+    int64_t t = g.blk[2 * blockIdx.x + 1] + (int64_t)(g.pre[qq] >> 32) + wave_incl_scan_i64(n) - n;
+    for (int s = 0; s < n; ++s, ++t)
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        const int e = a.edges[cfg * 3 * kMcMaxTris + 3 * s + r];
+        const int ax = e >> 2, e0 = e & 1, e1 = e >> 1 & 1;
+        // the owning point: offset 0 along the edge, (e0, e1) on the other two axes
+        const int di = ax == 0 ? 0 : e0, dj = ax == 0 ? e0 : (ax == 1 ? 0 : e1);
+        const int dk = ax == 2 ? 0 : e1;
+        uint64_t ex = 0, ey = 0, ez = 0, nb = 0, ni = 0, nj = 0;
+        int64_t first = 0;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y)
+            if (di == x && dj == y) {
+              ex = ed[x][y][0];
+              ey = ed[x][y][1];
+              ez = ed[x][y][2];
+              nb = m.n[x][y];
+              ni = m.n[x + 1][y];
+              nj = m.n[x][y + 1];
+              first = lane + dk < 64 ? v0[x][y] : v1[x][y];
+            }
+        int64_t vid;
+        if (lane + dk < 64) {
+          const uint64_t below = low_bits(lane + dk);
+          vid = first + __popcll(ex & below) + __popcll(ey & below) + __popcll(ez & below);
+          if (ax > 0) vid += ex >> (lane + dk) & 1;
+          if (ax > 1) vid += ey >> (lane + dk) & 1;
+        } else {
+          // the first point of the row's next word: no point of its group comes before it
+          vid = first;
+          if (ax > 0 && i + di + 1 < a.nx) vid += (nb ^ ni) & 1;
+          if (ax > 1 && j + dj + 1 < a.ny) vid += (nb ^ nj) & 1;
+        }
+        faces[3 * t + r] = vid;
+      }
+  }
+}
+
 }  // namespace vx
 
 using namespace vx;
@@ -338,8 +746,14 @@ int vx_extract_fields(const float* sdf, const int64_t* geom, const float* box, c
   a.n[2] = n2;
   a.scale = scale;
   a.u = u;
-  const dim3 grid((unsigned)cdiv(n2, 256), (unsigned)n1, (unsigned)n0);
-  k_extract_fields<<<grid, 256, 0, (hipStream_t)stream>>>(a);
+  const int64_t last = (int64_t)(a.g.X - 1) * a.g.sx + (int64_t)(a.g.Y - 1) * a.g.sy +
+                       (int64_t)(a.g.Z - 1) * a.g.sz;
+  if (last < ((int64_t)1 << 31))
+    k_extract_fields<<<dim3((unsigned)cdiv(n2, 256), (unsigned)cdiv(n1, kFieldRows), (unsigned)n0),
+                       256, 0, (hipStream_t)stream>>>(a);
+  else
+    k_extract_fields_wide<<<dim3((unsigned)cdiv(n2, 256), (unsigned)n1, (unsigned)n0), 256, 0,
+                            (hipStream_t)stream>>>(a);
   return launch_status("extract_fields");
 }
 
@@ -372,6 +786,65 @@ int vx_mc_emit(const float* u, int nx, int ny, int nz, float iso, const int8_t* 
   k_mc_emit<<<grid, 256, 0, (hipStream_t)stream>>>(a, vincl, tincl, bounds ? 1 : 0, b[0], b[1],
                                                    b[2], e[0], e[1], e[2], verts, faces);
   return launch_status("mc_emit");
+}
+
+// Workspace of vx_mc_classify: the lattice's bit words, the groups' prefixes and the blocks'
+// counts.
+static int mc_groups(int64_t nx, int64_t ny, int64_t nz, void* ws, McGroups& g, int64_t& blocks) {
+  VX_CHECK_ARG(nx >= 1 && ny >= 1 && nz >= 1 && nx <= 65535 && ny <= 65535,
+               "marching cubes: bad size");
+  g.words = cdiv(nz, 64);
+  g.total = nx * ny * g.words;
+  blocks = cdiv(g.total, kMcThreads);
+  VX_CHECK_ARG(blocks <= 0x7fffffff, "marching cubes: field too large");
+  g.bits = (uint64_t*)ws;
+  g.pre = g.bits + g.total;
+  g.blk = (int64_t*)(g.pre + g.total);
+  return VX_OK;
+}
+
+int64_t vx_mc_workspace_bytes(int nx, int ny, int nz) {
+  McGroups g;
+  int64_t blocks;
+  if (mc_groups(nx, ny, nz, nullptr, g, blocks)) return -1;
+  return 8 * (2 * g.total + 2 * blocks);
+}
+
+int vx_mc_classify(const float* u, int nx, int ny, int nz, float iso, const int8_t* count,
+                   void* ws, int64_t* totals, void* stream) {
+  VX_CHECK_ARG(u && count && ws && totals, "mc_classify: missing argument");
+  McGroups g;
+  int64_t blocks;
+  if (int e = mc_groups(nx, ny, nz, ws, g, blocks)) return e;
+  hipStream_t st = (hipStream_t)stream;
+  McArgs a{u, nx, ny, nz, iso, count, nullptr};
+  k_mc_below<<<grid_for(g.total, 32, 8192), 256, 0, st>>>(u, nz, iso, g);
+  k_mc_groups<<<(unsigned)blocks, kMcThreads, 0, st>>>(a, g);
+  k_mc_scan<<<1, 1024, 0, st>>>(g.blk, blocks, totals);
+  return launch_status("mc_classify");
+}
+
+int vx_mc_write(const float* u, int nx, int ny, int nz, float iso, const int8_t* count,
+                const int8_t* edges, void* ws, int64_t n_verts, int64_t n_faces,
+                const double* bounds, double* verts, int64_t* faces, void* stream) {
+  VX_CHECK_ARG(u && count && edges && ws && verts && faces, "mc_write: missing argument");
+  VX_CHECK_ARG(n_verts >= 0 && n_faces >= 0, "mc_write: negative size");
+  if (n_verts == 0) return VX_OK;
+  McGroups g;
+  int64_t blocks;
+  if (int e = mc_groups(nx, ny, nz, ws, g, blocks)) return e;
+  McArgs a{u, nx, ny, nz, iso, count, edges};
+  McWorld wd{};
+  wd.on = bounds != nullptr;
+  // float32 bounds, their difference taken in float32, as vx_mc_emit
+  if (bounds)
+    for (int i = 0; i < 3; ++i) {
+      wd.bmin[i] = (double)(float)bounds[i];
+      wd.ext[i] = (double)((float)bounds[3 + i] - (float)bounds[i]);
+    }
+  k_mc_write<<<(unsigned)blocks, kMcThreads, 0, (hipStream_t)stream>>>(a, g, wd, n_verts, n_faces,
+                                                                      verts, faces);
+  return launch_status("mc_write");
 }
 
 }  // extern "C"

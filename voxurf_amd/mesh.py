@@ -14,7 +14,7 @@ threshold 0 (what the reference meshes) that is outward.
 import numpy as np
 import torch
 
-from ._lib import call, lib, ptr, stream_of
+from ._lib import VoxhipError, call, lib, ptr, stream_of
 from .total_variation_cuda import grid_geom
 
 _TABLES = {}
@@ -66,26 +66,22 @@ def marching_cubes(u, threshold=0.0, bound_min=None, bound_max=None):
     dev = u.device
     st = stream_of(u)
     count, edges = _tables(dev)
-    n = nx * ny * nz
-    vcnt = torch.empty(n, dtype=torch.int64, device=dev)
-    tcnt = torch.empty(n, dtype=torch.int64, device=dev)
-    call("vx_mc_count", ptr(u), nx, ny, nz, float(threshold), ptr(count), ptr(edges), ptr(vcnt),
-         ptr(tcnt), st)
-    ws = torch.empty(max(1, lib().vx_scan_workspace_elems(n)), dtype=torch.int64, device=dev)
-    vincl = torch.empty_like(vcnt)
-    tincl = torch.empty_like(tcnt)
-    call("vx_inclusive_scan_i64", ptr(vcnt), ptr(vincl), n, ptr(ws), st)
-    call("vx_inclusive_scan_i64", ptr(tcnt), ptr(tincl), n, ptr(ws), st)
-    totals = torch.stack([vincl[-1], tincl[-1]]).tolist()
-    nv, nf = int(totals[0]), int(totals[1])
+    need = lib().vx_mc_workspace_bytes(nx, ny, nz)
+    if need < 0:
+        raise VoxhipError(lib().vx_last_error().decode())
+    ws = torch.empty(need // 8, dtype=torch.int64, device=dev)
+    totals = torch.empty(2, dtype=torch.int64, device=dev)
+    call("vx_mc_classify", ptr(u), nx, ny, nz, float(threshold), ptr(count), ptr(ws), ptr(totals),
+         st)
+    nv, nf = totals.tolist()
     verts = torch.empty((max(nv, 1), 3), dtype=torch.float64, device=dev)
     faces = torch.empty((max(nf, 1), 3), dtype=torch.int64, device=dev)
     bounds = None
     if bound_min is not None:
         bounds = np.asarray([*torch.as_tensor(bound_min).tolist(),
                              *torch.as_tensor(bound_max).tolist()], dtype=np.float64)
-    call("vx_mc_emit", ptr(u), nx, ny, nz, float(threshold), ptr(count), ptr(edges), ptr(vincl),
-         ptr(tincl), None if bounds is None else bounds.ctypes.data, ptr(verts), ptr(faces), st)
+    call("vx_mc_write", ptr(u), nx, ny, nz, float(threshold), ptr(count), ptr(edges), ptr(ws), nv, nf,
+         None if bounds is None else bounds.ctypes.data, ptr(verts), ptr(faces), st)
     return verts[:nv], faces[:nf]
 
 
