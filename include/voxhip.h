@@ -230,6 +230,21 @@ int vx_view_hit_coarse_geo(const float* cam, const float* box, const float* para
                            const float* mc, const int64_t* mc_geom, const float* mc_params,
                            int64_t* flag, void* stream);
 
+/* Occupancy of a MaskCache: which bricks and blocks of its grid hold a sample that could pass
+ * (vx_maskcache_occupancy_bytes bytes, 8-byte aligned; -1: bad geometry).  The _occ forms of
+ * the two entries above take it (or NULL) and give the same flags, jumping over what is
+ * clear; it must be that of the same mc, mc_geom and mc_params. */
+int64_t vx_maskcache_occupancy_bytes(const int64_t* mc_geom);
+int vx_maskcache_occupancy(const float* mc, const int64_t* mc_geom, const float* mc_params,
+                           void* occ, void* stream);
+int vx_hit_coarse_geo_occ(const float* rays_o, const float* rays_d, int64_t n_rays,
+                          const float* box, const float* params, const float* mc,
+                          const int64_t* mc_geom, const float* mc_params, const void* occ,
+                          uint8_t* hit, int64_t* flag, void* stream);
+int vx_view_hit_coarse_geo_occ(const float* cam, const float* box, const float* params,
+                               const float* mc, const int64_t* mc_geom, const float* mc_params,
+                               const void* occ, int64_t* flag, void* stream);
+
 /* lib/voxurf_fine.py:1150-1155 (img[mask], rays_o[mask], ...): incl = inclusive scan of
  * the view's flags; kept pixels are written in pixel order to rows incl[p] - 1 of
  * rgb_out, o_out, d_out, v_out [*, 3] (rgb [H*W, 3] float32). */
@@ -292,7 +307,7 @@ int vx_mc_emit(const float* u, int nx, int ny, int nz, float iso, const int8_t* 
                const double* bounds, double* verts, int64_t* faces, void* stream);
 
 /* Marching cubes of the whole field in two calls: vx_mc_classify fills the workspace `ws`
- * (vx_mc_workspace_bytes, 8-byte aligned; -1: sizes out of range) and totals = {vertices,
+ * (vx_mc_workspace_bytes, 16-byte aligned; -1: sizes out of range) and totals = {vertices,
  * triangles} (device); vx_mc_write, with those totals, the mesh vx_mc_emit writes (same
  * vertices, triangles and order).  u, iso and ws must be the classify call's. */
 int64_t vx_mc_workspace_bytes(int nx, int ny, int nz);

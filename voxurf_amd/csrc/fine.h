@@ -47,24 +47,35 @@ __device__ __forceinline__ bool skip_sample(const FusedGeom& G, const float q[3]
   return (b.x * (1.f - 1e-6f) - hfac * b.y) * G.inv_s >= G.skip_xmin;
 }
 
-// MaskCache.forward for one point (lib/voxurf_fine.py:930-942), as vx_maskcache_alpha.
-__device__ __forceinline__ bool maskcache_pass(const FusedGeom& G, const float q[3]) {
-#pragma clang fp contract(off)
-  const float fx = world_to_index(q[0], G.mc_mn[0], G.mc_mx[0] - G.mc_mn[0], G.gm.X);
-  const float fy = world_to_index(q[1], G.mc_mn[1], G.mc_mx[1] - G.mc_mn[1], G.gm.Y);
-  const float fz = world_to_index(q[2], G.mc_mn[2], G.mc_mx[2] - G.mc_mn[2], G.gm.Z);
-  float d;
+// MaskCache.forward for one point (lib/voxurf_fine.py:930-942), as vx_maskcache_alpha: the
+// density at a continuous index of the cache's grid, and whether its alpha passes.
+__device__ __forceinline__ void maskcache_index(const FusedGeom& G, const float q[3], float f[3]) {
+  f[0] = world_to_index(q[0], G.mc_mn[0], G.mc_mx[0] - G.mc_mn[0], G.gm.X);
+  f[1] = world_to_index(q[1], G.mc_mn[1], G.mc_mx[1] - G.mc_mn[1], G.gm.Y);
+  f[2] = world_to_index(q[2], G.mc_mn[2], G.mc_mx[2] - G.mc_mn[2], G.gm.Z);
+}
+
+__device__ __forceinline__ float maskcache_density(const FusedGeom& G, const float f[3]) {
   if (G.mc_nearest) {
-    const int x = sat_f2i(rintf(fx)), y = sat_f2i(rintf(fy)), z = sat_f2i(rintf(fz));
-    d = in_grid<float>(x, y, z, G.gm) ? G.mc[x * G.gm.sx + y * G.gm.sy + z * G.gm.sz] : 0.f;
-  } else {
-    Tri<float> t;
-    t.init(fx, fy, fz);
-    d = tri_gather(G.mc, G.gm, t, 0);
+    const int x = sat_f2i(rintf(f[0])), y = sat_f2i(rintf(f[1])), z = sat_f2i(rintf(f[2]));
+    return in_grid<float>(x, y, z, G.gm) ? G.mc[x * G.gm.sx + y * G.gm.sy + z * G.gm.sz] : 0.f;
   }
+  Tri<float> t;
+  t.init(f[0], f[1], f[2]);
+  return tri_gather(G.mc, G.gm, t, 0);
+}
+
+__device__ __forceinline__ bool maskcache_alpha_pass(const FusedGeom& G, float d) {
+#pragma clang fp contract(off)
   const float x = d + G.mc_shift;
   const float sp = x > 20.f ? x : log1pf(expf(x));
   return 1.f - expf(-sp * G.mc_ratio) >= G.mc_thres;
+}
+
+__device__ __forceinline__ bool maskcache_pass(const FusedGeom& G, const float q[3]) {
+  float f[3];
+  maskcache_index(G, q, f);
+  return maskcache_alpha_pass(G, maskcache_density(G, f));
 }
 
 __device__ __forceinline__ void ray_setup(const FusedGeom& G, const float* o, const float* d,

@@ -92,6 +92,14 @@ def _prefilter_args(mask_cache, xyz_min, xyz_max, near, stepdist):
     return box, params, maskcache_args(mask_cache)
 
 
+def _occupancy(mask_cache, mc):
+    """The MaskCache's occupancy (vx_maskcache_occupancy) for one call's walks."""
+    need = lib().vx_maskcache_occupancy_bytes(mc[1])
+    occ = torch.empty(max(1, need), dtype=torch.uint8, device=mask_cache.density.device)
+    call("vx_maskcache_occupancy", *mc, ptr(occ), stream_of(mask_cache.density))
+    return occ
+
+
 def hit_coarse_geo(mask_cache, xyz_min, xyz_max, rays_o, rays_d, near, stepdist):
     """Whether each ray hits the coarse geometry (lib/voxurf_fine.py:579-591): some
     in-box sample (sample_pts_on_rays with far = 1e9) passes the MaskCache.  bool [...]."""
@@ -104,8 +112,9 @@ def hit_coarse_geo(mask_cache, xyz_min, xyz_max, rays_o, rays_d, near, stepdist)
         raise RuntimeError("hit_coarse_geo: rays_o and rays_d differ in shape")
     box, params, mc = _prefilter_args(mask_cache, xyz_min, xyz_max, near, stepdist)
     hit = torch.empty(o.shape[0], dtype=torch.bool, device=o.device)
-    call("vx_hit_coarse_geo", ptr(o), ptr(d), o.shape[0], box.data_ptr(), params.data_ptr(),
-         *mc, ptr(hit), None, stream_of(o))
+    occ = _occupancy(mask_cache, mc)
+    call("vx_hit_coarse_geo_occ", ptr(o), ptr(d), o.shape[0], box.data_ptr(), params.data_ptr(),
+         *mc, ptr(occ), ptr(hit), None, stream_of(o))
     return hit.reshape(shape)
 
 
@@ -126,10 +135,12 @@ def get_training_rays_in_maskcache_sampling(rgb_tr_ori, train_poses, HW, Ks, ndc
     box, params, mc = _prefilter_args(model.mask_cache, model.xyz_min, model.xyz_max,
                                       render_kwargs["near"], stepdist)
     N = sum(im.shape[0] * im.shape[1] for im in rgb_tr_ori)
-    rgb_tr = torch.zeros([N, 3], device=dev)
-    rays_o_tr = torch.zeros_like(rgb_tr)
-    rays_d_tr = torch.zeros_like(rgb_tr)
-    viewdirs_tr = torch.zeros_like(rgb_tr)
+    # (only the rows written below are returned)
+    rgb_tr = torch.empty([N, 3], device=dev)
+    rays_o_tr = torch.empty_like(rgb_tr)
+    rays_d_tr = torch.empty_like(rgb_tr)
+    viewdirs_tr = torch.empty_like(rgb_tr)
+    occ = _occupancy(model.mask_cache, mc)
     imsz = []
     top = 0
     st = stream_of(rgb_tr)
@@ -138,8 +149,8 @@ def get_training_rays_in_maskcache_sampling(rgb_tr_ori, train_poses, HW, Ks, ndc
         cam = camera_params(H, W, K, c2w, inverse_y, flip_x, flip_y, "center", ndc)
         n = H * W
         flag = torch.empty(n, dtype=torch.int64, device=dev)
-        call("vx_view_hit_coarse_geo", cam.data_ptr(), box.data_ptr(), params.data_ptr(), *mc,
-             ptr(flag), st)
+        call("vx_view_hit_coarse_geo_occ", cam.data_ptr(), box.data_ptr(), params.data_ptr(), *mc,
+             ptr(occ), ptr(flag), st)
         incl = torch.empty_like(flag)
         ws = torch.empty(max(1, lib().vx_scan_workspace_elems(n)), dtype=torch.int64, device=dev)
         call("vx_inclusive_scan_i64", ptr(flag), ptr(incl), n, ptr(ws), st)
