@@ -230,6 +230,13 @@ int vx_view_hit_coarse_geo(const float* cam, const float* box, const float* para
                            const float* mc, const int64_t* mc_geom, const float* mc_params,
                            int64_t* flag, void* stream);
 
+/* SDF and unit normal grad / (|grad| + 1e-5) of the 6-neighbour gradient at the tile^3 points
+ * -1 + 2 (origin + i) / (res - 1) of a res^3 lattice (lib/dvgo_ori.py:679-693 with
+ * lib/voxurf_fine.py:502-534); box = {xyz_min, xyz_max} and origin[3] in host memory; out
+ * [tile^3], normal [tile^3, 3], z fastest. */
+int vx_sdf_query(const float* sdf, const int64_t* geom, const float* box, float voxel_size,
+                 float res, const float* origin, int tile, float* out, float* normal, void* stream);
+
 /* Occupancy of a MaskCache: which bricks and blocks of its grid hold a sample that could pass
  * (vx_maskcache_occupancy_bytes bytes, 8-byte aligned; -1: bad geometry).  The _occ forms of
  * the two entries above take it (or NULL) and give the same flags, jumping over what is

@@ -29,6 +29,116 @@ __global__ void k_tri_fwd(const T* __restrict__ grid, GridDesc g, const T* __res
   }
 }
 
+// The same for channels-innermost grids (channel stride 1): a lane per point and V
+// neighbouring channels, 16-byte corner loads where C, the strides and the base allow V = 4
+// (or 8-byte ones, V = 2), so that a point's lanes read one run per corner and write one run.
+// A lane per point that looped over the channels read 64 scattered lines per load: 38 us for
+// 100 k points of a 256^3 x 12 grid, against 13 us here.  Each channel is summed as above.
+template <typename T, int V>
+struct alignas(V * sizeof(T)) ChanVec {
+  T v[V];
+};
+
+template <typename T, int V>
+__global__ void __launch_bounds__(256) k_tri_fwd_rows(const T* __restrict__ grid, GridDesc g,
+                                                      const T* __restrict__ xyz,
+                                                      const T* __restrict__ mn,
+                                                      const T* __restrict__ mx, int64_t n,
+                                                      T* __restrict__ out) {
+#pragma clang fp contract(off)
+  using Vec = ChanVec<T, V>;
+  const T ex = mx[0] - mn[0], ey = mx[1] - mn[1], ez = mx[2] - mn[2];
+  const int cv = g.C / V;
+  const int64_t total = n * cv;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t p = total <= 0x7fffffff ? (int64_t)((uint32_t)i / (uint32_t)cv) : i / cv;
+    const int c = (int)(i - p * cv) * V;
+    Tri<T> t;
+    t.init(world_to_index(xyz[3 * p], mn[0], ex, g.X), world_to_index(xyz[3 * p + 1], mn[1], ey, g.Y),
+           world_to_index(xyz[3 * p + 2], mn[2], ez, g.Z));
+    Vec v[8];
+    bool in[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int x = t.x0 + (k >> 2), y = t.y0 + (k >> 1 & 1), z = t.z0 + (k & 1);
+      in[k] = in_grid<T>(x, y, z, g);
+      v[k] = *reinterpret_cast<const Vec*>(grid + c + clamp_index(x, g.X) * g.sx +
+                                           clamp_index(y, g.Y) * g.sy + clamp_index(z, g.Z) * g.sz);
+    }
+    Vec acc;
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc.v[e] = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (!in[k]) continue;
+      const T w = t.w(k >> 2, k >> 1 & 1, k & 1);
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc.v[e] += v[k].v[e] * w;
+    }
+    *reinterpret_cast<Vec*>(out + p * g.C + c) = acc;
+  }
+}
+
+// Its adjoint: L lanes per point (the power of two that holds the channels), a lane per
+// channel, so that an atomic instruction's lanes hit one run per point.  Consecutive points
+// (a ray's samples, half a voxel apart) often share their cell: the 64 / L points of a pass
+// that do add their corner terms across the lane groups first, and the first of them issues
+// the atomics.  Bound by the rate of scattered atomic requests: a lane per point and its own
+// 8 C atomics took 480 us for 100 k points x 12 channels, this 44 us.
+template <typename T, int L>
+__global__ void __launch_bounds__(256) k_tri_bwd_rows(T* __restrict__ grad, GridDesc g,
+                                                      const T* __restrict__ xyz,
+                                                      const T* __restrict__ mn,
+                                                      const T* __restrict__ mx, int64_t n,
+                                                      const T* __restrict__ gout) {
+#pragma clang fp contract(off)
+  constexpr int P = 64 / L;  // points per pass
+  const T ex = mx[0] - mn[0], ey = mx[1] - mn[1], ez = mx[2] - mn[2];
+  const int lane = threadIdx.x & 63, grp = lane / L, ch = lane % L;
+  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  for (int64_t base = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * P; base < n;
+       base += waves * P) {
+    const int64_t p = base + grp;
+    const bool valid = p < n;
+    const int64_t q = valid ? p : n - 1;
+    Tri<T> t;
+    t.init(world_to_index(xyz[3 * q], mn[0], ex, g.X), world_to_index(xyz[3 * q + 1], mn[1], ey, g.Y),
+           world_to_index(xyz[3 * q + 2], mn[2], ez, g.Z));
+    const T go = valid && ch < g.C ? gout[q * g.C + ch] : (T)0;
+    T v[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) v[b] = go == (T)0 ? (T)0 : t.w(b >> 2, (b >> 1) & 1, b & 1) * go;
+    // runs of points in one cell among the pass's groups
+    const int px = __shfl(t.x0, (lane - L) & 63, 64), py = __shfl(t.y0, (lane - L) & 63, 64),
+              pz = __shfl(t.z0, (lane - L) & 63, 64);
+    const bool same = grp > 0 && valid && px == t.x0 && py == t.y0 && pz == t.z0;
+    const uint64_t heads = __ballot(!same);
+    if (heads != ~0ull) {
+      // the run of this group ends before the next head
+      const uint64_t later = lane - ch + L < 64 ? heads >> (lane - ch + L) << (lane - ch + L) : 0;
+      const int end = later ? __ffsll((unsigned long long)later) - 1 : 64;  // first lane of it
+#pragma unroll
+      for (int off = L; off < 64; off <<= 1) {
+        const bool take = lane + off < end;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+          const T o = __shfl_down(v[b], off, 64);
+          if (take) v[b] += o;
+        }
+      }
+    }
+    if (valid && !same && ch < g.C) {
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const int x = t.x0 + (b >> 2), y = t.y0 + ((b >> 1) & 1), z = t.z0 + (b & 1);
+        if (v[b] != (T)0 && in_grid<T>(x, y, z, g))
+          atomic_add(&grad[ch + x * g.sx + y * g.sy + z * g.sz], v[b]);
+      }
+    }
+  }
+}
+
 template <typename T>
 __global__ void k_tri_bwd(T* __restrict__ grad, GridDesc g, const T* __restrict__ xyz,
                           const T* __restrict__ mn, const T* __restrict__ mx, int64_t n,
@@ -163,6 +273,101 @@ __global__ void k_sdf_grad_bwd(T* __restrict__ ggrid, GridDesc g, const T* __res
   }
 }
 
+// The adjoint without the neighbour values' gradients (gfeat), for consecutive samples of
+// rays.  A sample adds to 32 voxels (sdf7_terms): as 32 atomics of a lane they are 32
+// scattered requests, and the rate of those bounds the scatter (359 us for the 1.5 M samples
+// of a coarse step, of which one in six has a gradient).  Here a wave leaves its samples'
+// terms in LDS, and half a wave takes a run of samples in one cell, a lane per voxel: the
+// run's terms are added first, and the voxels of a z line (12 lines per cell) go out as one
+// request.  Measured 136 us.
+constexpr int kScatterThreads = 256;
+template <typename T>
+__global__ void __launch_bounds__(kScatterThreads) k_sdf_grad_bwd_runs(
+    T* __restrict__ ggrid, GridDesc g, const T* __restrict__ xyz, const T* __restrict__ mn,
+    const T* __restrict__ mx, T voxel_size, int64_t n, const T* __restrict__ gsdf,
+    const T* __restrict__ ggrad) {
+#pragma clang fp contract(off)
+  constexpr int kStride = 33;  // odd: the lanes' rows spread over the banks
+  __shared__ T terms[kScatterThreads * kStride];
+  __shared__ int cell[kScatterThreads * 3];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, vl = lane & 31;
+  T* tw = terms + wave * 64 * kStride;
+  int* cw = cell + wave * 64 * 3;
+  // this lane's voxel of a cell's 32 (offsets from the cell): the order of Sdf7Terms
+  int dx, dy, dz;
+  if (vl < 8) {
+    dx = vl >> 2;
+    dy = vl >> 1 & 1;
+    dz = vl & 1;
+  } else {
+    const int c = (vl - 8) >> 3, side = (vl >> 2) & 1, j = vl & 3;
+    const int lo = c == 0 ? 1 : 0, hi = c == 2 ? 1 : 2;
+    int v[3] = {0, 0, 0};
+    v[c] = side ? 2 : -1;
+    v[lo] += j >> 1;
+    v[hi] += j & 1;
+    dx = v[0];
+    dy = v[1];
+    dz = v[2];
+  }
+  const int64_t waves = (int64_t)gridDim.x * (kScatterThreads >> 6);
+  for (int64_t base = ((int64_t)blockIdx.x * (kScatterThreads >> 6) + wave) * 64; base < n;
+       base += waves * 64) {
+    const int64_t p = base + lane;
+    const T gs = p < n && gsdf ? gsdf[p] : (T)0;
+    const T gg[3] = {p < n && ggrad ? ggrad[3 * p] : (T)0, p < n && ggrad ? ggrad[3 * p + 1] : (T)0,
+                     p < n && ggrad ? ggrad[3 * p + 2] : (T)0};
+    const bool act = gs != (T)0 || gg[0] != (T)0 || gg[1] != (T)0 || gg[2] != (T)0;
+    const uint64_t acts = __ballot(act);
+    if (acts == 0) continue;
+    int x0 = 0, y0 = 0, z0 = 0;
+    if (act) {
+      const T q[3] = {xyz[3 * p], xyz[3 * p + 1], xyz[3 * p + 2]};
+      Sdf7Terms<T> o;
+      sdf7_terms(ggrid, g, q, mn, mx, voxel_size, gs, gg, o);
+      x0 = o.x0;
+      y0 = o.y0;
+      z0 = o.z0;
+      T* row = tw + lane * kStride;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) row[b] = o.acc[b];
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int sd = 0; sd < 2; ++sd)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) row[8 + 8 * c + 4 * sd + j] = o.out[c][sd][j];
+      cw[3 * lane] = x0;
+      cw[3 * lane + 1] = y0;
+      cw[3 * lane + 2] = z0;
+    }
+    const int px = __shfl_up(x0, 1, 64), py = __shfl_up(y0, 1, 64), pz = __shfl_up(z0, 1, 64);
+    const bool prev = lane > 0 && (acts >> (lane - 1) & 1);
+    const bool head = act && !(prev && px == x0 && py == y0 && pz == z0);
+    // runs: from each head up to the next head or gap
+    const uint64_t heads = __ballot(head), stops = heads | ~acts;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the terms, for the other lanes
+    uint64_t todo = heads;
+    while (todo) {
+      // one run for each half of the wave
+      const int first = __ffsll((unsigned long long)todo) - 1;
+      todo &= todo - 1;
+      const int second = todo ? __ffsll((unsigned long long)todo) - 1 : -1;
+      todo &= todo - 1;
+      const int r = half ? second : first;
+      if (r < 0) continue;
+      const uint64_t after = r < 63 ? stops >> (r + 1) : 0;
+      const int end = after ? r + __ffsll((unsigned long long)after) : 64;
+      T sum = tw[r * kStride + vl];
+      for (int k = r + 1; k < end; ++k) sum += tw[k * kStride + vl];
+      const int x = cw[3 * r] + dx, y = cw[3 * r + 1] + dy, z = cw[3 * r + 2] + dz;
+      if (sum != (T)0 && in_grid<T>(x, y, z, g))
+        atomic_add(&ggrid[x * g.sx + y * g.sy + z * g.sz], sum);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+}
+
 // ---- neus_sdf_gradient 'interpolate' (lib/voxurf_fine.py:440-450) ------------------
 // out[a] = (s[+1] - s[-1]) / 2 / voxel_size along axis a, 0 on that axis' boundary faces.
 // Launched as a 3-D grid (z chunks of 256 threads, y, x): no index division.
@@ -240,6 +445,34 @@ __global__ void k_tv(const T* __restrict__ param, T* __restrict__ grad, const T*
     term(i < g.X - 1, a + g.sx, wi);
     grad[a] += (T)add;
   }
+}
+
+// ---- SDF and unit normal on a lattice tile (lib/dvgo_ori.py:679-693 with the normal of
+// lib/voxurf_fine.py:502-534) --------------------------------------------------------------
+// One thread per point of the tile (3-D launch: z chunks of 64, y, x), its lattice point
+// (-1 + 2 i / (res - 1) per axis, as a product with the reciprocal) made in registers; normal = grad / (|grad| + 1e-5).
+struct QueryArgs {
+  const float* sdf;
+  GridDesc g;
+  float mn[3], mx[3], voxel_size, step;  // step: 1 / (res - 1)
+  float o[3];
+  int tile;
+  float* out;
+  float* normal;
+};
+
+__global__ void __launch_bounds__(64) k_sdf_query(QueryArgs a) {
+#pragma clang fp contract(off)
+  const int k = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y, i = blockIdx.z;
+  if (k >= a.tile) return;
+  const float q[3] = {-1.f + 2.f * ((float)i + a.o[0]) * a.step, -1.f + 2.f * ((float)j + a.o[1]) * a.step,
+                      -1.f + 2.f * ((float)k + a.o[2]) * a.step};
+  float s, gr[3];
+  sdf7<float>(a.sdf, a.g, q, a.mn, a.mx, a.voxel_size, s, gr, nullptr);
+  const int64_t p = ((int64_t)i * a.tile + j) * a.tile + k;
+  const float den = sqrtf(gr[0] * gr[0] + gr[1] * gr[1] + gr[2] * gr[2]) + 1e-5f;
+  a.out[p] = s;
+  for (int c = 0; c < 3; ++c) a.normal[3 * p + c] = gr[c] / den;
 }
 
 // ---- MaskCache.forward (lib/voxurf_fine.py:930-942, lib/dvgo_ori.py:440-473) --------
@@ -321,6 +554,48 @@ static int make_desc(const int64_t* shape_strides, GridDesc& g) {
 #define CP(p) ((const scalar_t*)(p))
 #define MP(p) ((scalar_t*)(p))
 
+// Channels per lane of the channels-innermost lookup: as many as one aligned load of up to 16
+// bytes takes, given the channel count, the strides and the bases.
+template <typename T>
+static int row_vec(const GridDesc& g, const void* grid, const void* out) {
+  for (int v = 16 / (int)sizeof(T); v > 1; v /= 2) {
+    const uintptr_t bytes = (uintptr_t)v * sizeof(T);
+    if (g.C % v == 0 && g.sx % v == 0 && g.sy % v == 0 && g.sz % v == 0 &&
+        (uintptr_t)grid % bytes == 0 && (uintptr_t)out % bytes == 0)
+      return v;
+  }
+  return 1;
+}
+
+template <typename T>
+static void tri_fwd_rows(const T* grid, const GridDesc& g, const T* xyz, const T* mn, const T* mx,
+                         int64_t n, T* out, hipStream_t st) {
+  const int v = row_vec<T>(g, grid, out);
+  const unsigned blocks = grid_for(n * (g.C / v), 256);
+  if (v == 4) {
+    if constexpr (sizeof(T) == 4)
+      k_tri_fwd_rows<T, 4><<<blocks, 256, 0, st>>>(grid, g, xyz, mn, mx, n, out);
+  } else if (v == 2) {
+    k_tri_fwd_rows<T, 2><<<blocks, 256, 0, st>>>(grid, g, xyz, mn, mx, n, out);
+  } else {
+    k_tri_fwd_rows<T, 1><<<blocks, 256, 0, st>>>(grid, g, xyz, mn, mx, n, out);
+  }
+}
+
+template <typename T>
+static void tri_bwd_rows(T* grad, const GridDesc& g, const T* xyz, const T* mn, const T* mx,
+                         int64_t n, const T* gout, hipStream_t st) {
+#define VX_TRI_BWD(L) \
+  k_tri_bwd_rows<T, L><<<grid_for(cdiv(n, 64 / L), 4), 256, 0, st>>>(grad, g, xyz, mn, mx, n, gout)
+  if (g.C <= 2) VX_TRI_BWD(2);
+  else if (g.C <= 4) VX_TRI_BWD(4);
+  else if (g.C <= 8) VX_TRI_BWD(8);
+  else if (g.C <= 16) VX_TRI_BWD(16);
+  else if (g.C <= 32) VX_TRI_BWD(32);
+  else VX_TRI_BWD(64);
+#undef VX_TRI_BWD
+}
+
 extern "C" {
 
 int vx_grid_sample_fwd(int dtype, const void* grid, const int64_t* geom, const void* xyz,
@@ -330,6 +605,12 @@ int vx_grid_sample_fwd(int dtype, const void* grid, const int64_t* geom, const v
   if (int st = make_desc(geom, g)) return st;
   VX_CHECK_ARG(n >= 0, "grid_sample: n < 0");
   if (n == 0) return VX_OK;
+  // channels innermost: lanes over a point's channels (other orders: a lane per point)
+  if (g.C > 1 && g.sc == 1) {
+    GRID_DISPATCH(dtype, tri_fwd_rows<scalar_t>(CP(grid), g, CP(xyz), CP(xyz_min), CP(xyz_max), n,
+                                                MP(out), ST(stream)));
+    return launch_status("grid_sample_fwd");
+  }
   GRID_DISPATCH(dtype, k_tri_fwd<scalar_t><<<grid_for(n, 256), 256, 0, ST(stream)>>>(
                            CP(grid), g, CP(xyz), CP(xyz_min), CP(xyz_max), n, MP(out)));
   return launch_status("grid_sample_fwd");
@@ -342,6 +623,12 @@ int vx_grid_sample_bwd(int dtype, void* grad, const int64_t* geom, const void* x
   if (int st = make_desc(geom, g)) return st;
   VX_CHECK_ARG(n >= 0, "grid_sample: n < 0");
   if (n == 0) return VX_OK;
+  // channels innermost, at most a wave's lanes of them: lanes over a point's channels
+  if (g.C > 1 && g.C <= 64 && g.sc == 1) {
+    GRID_DISPATCH(dtype, tri_bwd_rows<scalar_t>(MP(grad), g, CP(xyz), CP(xyz_min), CP(xyz_max), n,
+                                                CP(gout), ST(stream)));
+    return launch_status("grid_sample_bwd");
+  }
   GRID_DISPATCH(dtype, k_tri_bwd<scalar_t><<<grid_for(n, 256), 256, 0, ST(stream)>>>(
                            MP(grad), g, CP(xyz), CP(xyz_min), CP(xyz_max), n, CP(gout)));
   return launch_status("grid_sample_bwd");
@@ -399,6 +686,14 @@ int vx_sdf_grad_bwd(int dtype, void* ggrid, const int64_t* geom, const void* xyz
   VX_CHECK_ARG(g.C == 1, "sdf_grad: the SDF grid must have one channel");
   VX_CHECK_ARG(n >= 0, "sdf_grad: n < 0");
   if (n == 0) return VX_OK;
+  // (the neighbour values' gradients, which the renderer never has, go through the plain form)
+  if (!gfeat) {
+    GRID_DISPATCH(dtype, k_sdf_grad_bwd_runs<scalar_t>
+                  <<<grid_for(n, kScatterThreads), kScatterThreads, 0, ST(stream)>>>(
+                      MP(ggrid), g, CP(xyz), CP(xyz_min), CP(xyz_max), (scalar_t)voxel_size, n,
+                      CP(gsdf), CP(ggrad)));
+    return launch_status("sdf_grad_bwd");
+  }
   GRID_DISPATCH(dtype, k_sdf_grad_bwd<scalar_t><<<grid_for(n, 256), 256, 0, ST(stream)>>>(
                            MP(ggrid), g, CP(xyz), CP(xyz_min), CP(xyz_max), (scalar_t)voxel_size,
                            n, CP(gsdf), CP(ggrad), CP(gfeat)));
@@ -453,6 +748,29 @@ int vx_total_variation_add_grad_new(int dtype, const void* param, void* grad, co
   GRID_DISPATCH(dtype, k_tv<scalar_t, true><<<grid_for(N, 256), 256, 0, ST(stream)>>>(
                            CP(param), MP(grad), CP(mask), g, wx, wy, wz, dense_mode));
   return launch_status("total_variation_add_grad_new");
+}
+
+int vx_sdf_query(const float* sdf, const int64_t* geom, const float* box, float voxel_size,
+                 float res, const float* origin, int tile, float* out, float* normal, void* stream) {
+  VX_CHECK_ARG(sdf && geom && box && origin && out && normal, "sdf_query: missing argument");
+  QueryArgs a;
+  if (int st = make_desc(geom, a.g)) return st;
+  VX_CHECK_ARG(a.g.C == 1, "sdf_query: the SDF grid must have one channel");
+  VX_CHECK_ARG(tile >= 0 && tile <= 65535, "sdf_query: bad tile size");
+  if (tile == 0) return VX_OK;
+  a.sdf = sdf;
+  for (int i = 0; i < 3; ++i) {
+    a.mn[i] = box[i];
+    a.mx[i] = box[3 + i];
+    a.o[i] = origin[i];
+  }
+  a.voxel_size = voxel_size;
+  a.step = 1.f / (res - 1.f);
+  a.tile = tile;
+  a.out = out;
+  a.normal = normal;
+  k_sdf_query<<<dim3((unsigned)cdiv(tile, 64), (unsigned)tile, (unsigned)tile), 64, 0, ST(stream)>>>(a);
+  return launch_status("sdf_query");
 }
 
 int vx_maskcache_alpha(int dtype, const void* density, const int64_t* geom, const void* xyz,

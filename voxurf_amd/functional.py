@@ -75,6 +75,7 @@ class SdfGradSample(torch.autograd.Function):
         call("vx_sdf_grad_fwd", dtype_code(grid), ptr(grid), geom.data_ptr(), ptr(xyz), ptr(mn),
              ptr(mx), float(voxel_size), n, ptr(sdf), ptr(grad), ptr(feat), stream_of(grid))
         ctx.save_for_backward(xyz, mn, mx)
+        ctx.set_materialize_grads(False)  # outputs nobody used have no gradient to scatter
         ctx.geom = geom
         ctx.vs = float(voxel_size)
         ctx.grid_like = grid
@@ -86,9 +87,9 @@ class SdfGradSample(torch.autograd.Function):
         xyz, mn, mx = ctx.saved_tensors
         grid = ctx.grid_like
         ggrid = _zeros_like_grid(grid)
-        c = lambda t: None if t is None else t.contiguous()  # noqa: E731
+        gsdf, ggrad, gfeat = (None if t is None else t.contiguous() for t in (gsdf, ggrad, gfeat))
         call("vx_sdf_grad_bwd", dtype_code(grid), ptr(ggrid), ctx.geom.data_ptr(), ptr(xyz),
-             ptr(mn), ptr(mx), ctx.vs, xyz.shape[0], ptr(c(gsdf)), ptr(c(ggrad)), ptr(c(gfeat)),
+             ptr(mn), ptr(mx), ctx.vs, xyz.shape[0], ptr(gsdf), ptr(ggrad), ptr(gfeat),
              stream_of(grid))
         return ggrid, None, None, None, None
 
@@ -120,10 +121,10 @@ class SampleSdfs(torch.autograd.Function):
     def backward(ctx, gfeat, ggrad):
         grid, xyz, mn, mx, disp = ctx.saved_tensors
         ggrid = _zeros_like_grid(grid)
-        c = lambda t: None if t is None else t.contiguous()  # noqa: E731
+        gfeat, ggrad = (None if t is None else t.contiguous() for t in (gfeat, ggrad))
         call("vx_sample_sdfs_bwd", dtype_code(grid), ptr(ggrid), ptr(grid), ctx.geom.data_ptr(),
              ptr(xyz), ptr(mn), ptr(mx), ptr(disp), disp.numel(), ctx.vs, ctx.norm, xyz.shape[0],
-             ptr(c(gfeat)), ptr(c(ggrad)), stream_of(grid))
+             ptr(gfeat), ptr(ggrad), stream_of(grid))
         return ggrid, None, None, None, None, None, None
 
 

@@ -170,18 +170,13 @@ class ResidentScene:
     def sdf_query(self, res, tile_origin, tile=64):
         """SDF and unit normal at a tile of the res^3 lattice over the bbox
         (x_i = -1 + 2 i / (res - 1)): points [tile^3, 3] -> (sdf [P], normal [P, 3])."""
-        i0, j0, k0 = tile_origin
-        ax = [(-1.0 + 2.0 * (torch.arange(tile, device=self.dev, dtype=torch.float32) + o) / (res - 1))
-              for o in (i0, j0, k0)]
-        X, Y, Z = torch.meshgrid(*ax, indexing="ij")
-        pts = torch.stack([X, Y, Z], -1).reshape(-1, 3).contiguous()
-        n = pts.shape[0]
+        origin = torch.tensor([float(v) for v in tile_origin], dtype=torch.float32)
+        n = tile ** 3
         sdf = torch.empty(n, dtype=torch.float32, device=self.dev)
-        grad = torch.empty((n, 3), dtype=torch.float32, device=self.dev)
-        call("vx_sdf_grad_fwd", 0, ptr(self.sdf), self.sdf_geom.data_ptr(), ptr(pts),
-             ptr(self.xyz_min), ptr(self.xyz_max), float(self.cfg.voxel_size), n, ptr(sdf),
-             ptr(grad), None, stream_of(pts))
-        normal = grad / (grad.norm(dim=-1, keepdim=True) + 1e-5)
+        normal = torch.empty((n, 3), dtype=torch.float32, device=self.dev)
+        call("vx_sdf_query", ptr(self.sdf), self.sdf_geom.data_ptr(), self.box.data_ptr(),
+             float(self.cfg.voxel_size), float(res), origin.data_ptr(), int(tile), ptr(sdf),
+             ptr(normal), stream_of(self.sdf))
         return sdf, normal
 
 
