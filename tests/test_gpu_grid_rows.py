@@ -1,5 +1,6 @@
 """The row forms of the grid operators (channels innermost, rows of z) against the general
-strided ones: the same bits where no sum is reordered (lookup, the lattice query), float64 to rounding where it is (the scatters); at the channel counts, strides, bases
+strided ones: the same bits where no sum is reordered (lookup, total variation, the lattice
+query), float64 to rounding where it is (the scatters); at the channel counts, strides, bases
 and sizes around the rules that choose them."""
 import pytest
 import torch
@@ -107,6 +108,42 @@ def test_sdf_gradient_without_neighbour_values(dev):
     s, gr, f = vf.SdfGradSample.apply(grid, pts, mn, mx, 0.2)
     gr.pow(2).sum().backward()                      # s and f without a gradient
     assert torch.allclose(grid.grad, outs[1], rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("C", [1, 3, 12])
+@pytest.mark.parametrize("inner", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 3, 5), (5, 1, 255), (3, 4, 256), (4, 5, 257)])
+@pytest.mark.parametrize("masked,dense", [(False, 1), (False, 0), (True, 1), (True, 0)])
+def test_total_variation_rows(dev, C, inner, shape, masked, dense):
+    g = torch.Generator().manual_seed(C + sum(shape))
+    X, Y, Z = shape
+    # the strided kernel gets the same values in rows one element longer
+    full = (X, Y, Z, C) if inner else (C, X, Y, Z)
+    val = [torch.randn(full, generator=g) for _ in range(3)]
+    val[1][torch.rand(full, generator=g) < 0.5] = 0
+    val[2] = (val[2] > 0).float()
+
+    def view(t, long):
+        if long:
+            w = torch.zeros((*full[:-1], full[-1] + 1))
+            w[..., :full[-1]] = t
+            t = w.to(dev)[..., :full[-1]]
+        else:
+            t = t.to(dev)
+        return (t.permute(3, 0, 1, 2) if inner else t)[None]
+
+    res = []
+    for long in (False, True):
+        p, gr, m = (view(v, long) for v in val)
+        geom = grid_geom(p)
+        if masked:
+            call("vx_total_variation_add_grad_new", 0, ptr(p), ptr(gr), ptr(m), geom.data_ptr(), 0.3,
+                 0.5, 0.7, dense, stream_of(p))
+        else:
+            call("vx_total_variation_add_grad", 0, ptr(p), ptr(gr), geom.data_ptr(), 0.3, 0.5, 0.7,
+                 dense, stream_of(p))
+        res.append(gr.contiguous())
+    assert torch.equal(*res)
 
 
 @pytest.mark.parametrize("tile,origin,res", [(1, (0, 0, 0), 8), (5, (3, 0, 2), 40), (63, (1, 4, 0), 70),
