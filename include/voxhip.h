@@ -547,6 +547,18 @@ int vx_mlp_layer_fwd(int prec, int kt, int k_in, int last, const void* in, int i
                      int64_t M, const void* wpk, const float* bias, void* out, int out_stride,
                      const float* w3, const float* b3, float* logits, const int64_t* M_dev,
                      uint32_t* mask_bits, void* stream);
+/* The whole network in one launch, FP32 accuracy from two-way FP16 splits of scaled rows and
+ * weights (three MFMA products per FP32 product).  vx_mlp_pack_half packs the hidden layers'
+ * weights (w_ptrs: host array of n_hidden device addresses, 1..4 layers, width 192, input
+ * width k_in0 <= 96) into vx_mlp_pack_half_bytes bytes (16-byte aligned; -1: bad sizes). */
+int64_t vx_mlp_pack_half_bytes(int n_hidden, int k_in0);
+int vx_mlp_pack_half(int n_hidden, const int64_t* w_ptrs, int k_in0, void* out, void* stream);
+/* logits [M, 3] of X [M, xs] (float32 rows padded to 64 columns for k_in0 <= 64, else 96;
+ * finite past k_in0) without keeping activations; biases: host array of n_hidden device
+ * addresses. */
+int vx_mlp_net_fwd(int n_hidden, int k_in0, const float* X, int xs, int64_t M, const void* packed,
+                   const int64_t* biases, const float* w3, const float* b3, float* logits,
+                   const int64_t* M_dev, void* stream);
 /* The 3-output layer alone: logits [M, 3] = W3 H + b3 from the last hidden activations
  * H [M, hs] (the last = 1 part of vx_mlp_layer_fwd). */
 int vx_mlp_logits(int prec, const void* H, int hs, int64_t M, const float* w3, const float* b3,

@@ -78,6 +78,27 @@ class Packed:
         self.prec = prec
 
 
+def _addresses(ts):
+    """Host array of device addresses."""
+    return torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64)
+
+
+def net_logits(X, Ws, bs, st, M_dev=None):
+    """logits [M, 3] of padded float32 rows X at split precision without keeping the hidden
+    activations: all layers in one launch, which never writes them (vx_mlp_net_fwd)."""
+    M, dev, n, k_in0 = X.shape[0], X.device, len(Ws) - 1, Ws[0].shape[1]
+    need = lib().vx_mlp_pack_half_bytes(n, k_in0)
+    if need < 0:
+        raise RuntimeError("rgbnet shape not supported by the MFMA kernels")
+    packed = torch.empty(need, dtype=torch.uint8, device=dev)
+    logits = torch.empty((M, 3), dtype=torch.float32, device=dev)
+    w_a, b_a = _addresses(Ws[:-1]), _addresses(bs[:-1])
+    call("vx_mlp_pack_half", n, w_a.data_ptr(), k_in0, ptr(packed), st)
+    call("vx_mlp_net_fwd", n, k_in0, ptr(X), X.shape[1], M, ptr(packed), b_a.data_ptr(),
+         ptr(Ws[-1]), ptr(bs[-1]), ptr(logits), ptr(M_dev), st)
+    return logits
+
+
 def forward_rows(X, Ws, bs, prec, packed, st, M_dev=None, timing=None, bits=None):
     """logits [M, 3] and the hidden activations of X [M, 32*kt0] (padded rows in the
     activation element type).  M_dev: optional device int64 row count (at most M rows of
@@ -276,13 +297,15 @@ def padded_rows(x, k_in, prec):
 
 class _MlpFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, prec, *params):
+    def forward(ctx, x, prec, keep, *params):
         Ws = [p.detach().contiguous() for p in params[0::2]]
         bs = [p.detach().contiguous() for p in params[1::2]]
         if any(w.dtype != torch.float32 for w in Ws):
             raise RuntimeError("rgbnet parameters must be float32")
         st = stream_of(x)
         X = padded_rows(x, Ws[0].shape[1], prec)
+        if prec == PREC_F32_SPLIT and not keep:
+            return net_logits(X, Ws, bs, st)
         packed = Packed(Ws, prec, st)
         bits = []
         logits, hs = forward_rows(X, Ws, bs, prec, packed, st, bits=bits)
@@ -301,7 +324,7 @@ class _MlpFn(torch.autograd.Function):
             grads += [torch.empty_like(W), torch.empty_like(b)]
         dX = backward_rows(X, hs, Ws, ctx.prec, ctx.packed, glogits.contiguous().float(),
                            stream_of(X), grads, bits=ctx.bits)
-        return (dX[:, :ctx.din], None, *grads)
+        return (dX[:, :ctx.din], None, None, *grads)
 
 
 def check_shapes(linears):
@@ -333,5 +356,7 @@ def mlp_forward(x, linears, compute_dtype=torch.float32, padded=False, f32_split
         if x.shape[-1] != linears[0].in_features:
             raise RuntimeError(f"rgbnet input width {x.shape[-1]} != {linears[0].in_features}")
         x2 = x.reshape(-1, x.shape[-1]).float()
-    out = _MlpFn.apply(x2, prec, *params)
+    # the activations are kept only for a gradient to come
+    keep = torch.is_grad_enabled() and (x2.requires_grad or any(p.requires_grad for p in params))
+    out = _MlpFn.apply(x2, prec, keep, *params)
     return out.reshape(*x.shape[:-1], 3)
