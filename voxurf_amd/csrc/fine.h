@@ -113,21 +113,6 @@ __device__ __forceinline__ void load_slot(const FusedGeom& G, const float* vd, f
   ss.w = ss.myT * ss.alpha;
 }
 
-// Position of the k-th set bit of m (k < popcount(m)).
-__device__ __forceinline__ int kth_set_bit(uint64_t m, int k) {
-  int pos = 0;
-#pragma unroll
-  for (int width = 32; width >= 1; width >>= 1) {
-    const uint64_t low = (m >> pos) & ((1ull << width) - 1ull);
-    const int c = __popcll(low);
-    if (k >= c) {
-      k -= c;
-      pos += width;
-    }
-  }
-  return pos;
-}
-
 // Host side: fill a FusedGeom from the C-ABI arguments.
 static inline int fused_geom(FusedGeom& G, const float* sdf, const int64_t* sdf_geom,
                              const float* k0, const int64_t* k0_geom, const float* box,
@@ -204,5 +189,12 @@ static inline int fused_maskcache(FusedGeom& G, const float* mc, const int64_t* 
   }
   return VX_OK;
 }
+
+// Survivor rows P4 = (x, y, z, weight), G4 = (gradient, sdf), rid of the walk-range slots
+// (k_survivors in fused.hip); n_rays > 0.
+void launch_survivors(const FusedGeom& G, const float* viewdirs, int64_t n_rays, int cap,
+                      const void* s4, const void* g4, const int* stats, const int64_t* cnt,
+                      const int64_t* off_incl, int64_t max_rows, void* P4, void* G4, int* rid,
+                      uint32_t* pages, hipStream_t st);
 
 }  // namespace vx

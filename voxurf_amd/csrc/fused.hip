@@ -220,119 +220,165 @@ __global__ void __launch_bounds__(256, 3) k_fused_fwd(
   }
 }
 
-// Compaction + rgbnet input.  One wavefront per ray takes its walk-range slots 64 at a
-// time, keeps the survivors (w > thres) at rows off[r] .. off[r] + cnt[r] and builds
-// X = [k0 (C) | normal (3) | view PE (3 + 6 nf) | 0 pad], four rows per pass with
-// sixteen lanes per row and four columns per lane.
+// Survivors (w > thres) of the walk-range slots: (x, y, z, w), (gradient, sdf) and the ray at
+// rows off[r] .. off[r] + cnt[r], sixteen lanes a ray.  What a row needs beyond that is built
+// by kernels over whole tiles of rows (k_fused_rows, k_voxurf_rows).  Both in one kernel, a
+// wavefront per ray, was bound by the instructions of half-empty wavefronts: a view embedding
+// per ray in sixteen of 64 lanes, both branches of sinf and cosf four columns deep (462 us of
+// a 131,072-ray render with 1.4 M rows, 41 at 1000 rays); in two: 29 + 140 us, and 4 + 7.
+__global__ void __launch_bounds__(256) k_survivors(
+    FusedGeom G, const float* __restrict__ viewdirs, int64_t n_rays, int cap,
+    const float4* __restrict__ s4, const float4* __restrict__ g4, const int* __restrict__ stats,
+    const int64_t* __restrict__ cnt, const int64_t* __restrict__ off_incl, int64_t max_rows,
+    float4* __restrict__ P4, float4* __restrict__ G4, int* __restrict__ rid,
+    uint32_t* __restrict__ pages) {
+  const int l = threadIdx.x & 15, sub = (threadIdx.x & 63) >> 4;
+  const int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 4) + (threadIdx.x >> 4);
+  int64_t c = 0, o = 0;
+  int c1 = 0;
+  float vd[3] = {0.f, 0.f, 0.f};
+  if (r < n_rays) {
+    c = cnt[r];
+    c1 = stats[3 * r + 1];
+    o = off_incl[r] - c;
+    for (int e = 0; e < 3; ++e) vd[e] = viewdirs[3 * r + e];
+    // past the output capacity nothing is written
+    if (c == 0 || (o >= max_rows && !pages)) c1 = 0;
+  }
+  int64_t ks = 0;
+  for (int base = 0; __any(base < c1 && ks < c); base += 16) {
+    const int k = base + l;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+    bool surv = false;
+    if (k < c1) {
+      a = s4[r * cap + k];
+      b = g4[r * cap + k];
+      SlotSample ss;
+      load_slot(G, vd, a, b, ss);
+      surv = ss.w > G.thres;
+      a.w = ss.w;
+    }
+    const uint32_t sm = (uint32_t)(__ballot(surv) >> (16 * sub)) & 0xffffu;
+    // rows past the forward's survivor count are never written (they cannot occur: the
+    // recomputed weights are the forward's)
+    const int64_t j = ks + __popc(sm & ((1u << l) - 1u));
+    if (surv && j < c) {
+      if (o + j < max_rows) {
+        P4[o + j] = a;
+        G4[o + j] = b;
+        rid[o + j] = (int)r;
+      }
+      if (pages) {
+        Tri<float> t;
+        t.init(world_to_index(a.x, G.mn[0], G.mx[0] - G.mn[0], G.gk.X),
+               world_to_index(a.y, G.mn[1], G.mx[1] - G.mn[1], G.gk.Y),
+               world_to_index(a.z, G.mn[2], G.mx[2] - G.mn[2], G.gk.Z));
+        for (int corner = 0; corner < 8; ++corner) mark_corner_pages(pages, G.gk, t, corner);
+      }
+    }
+    ks += __popc(sm);
+  }
+}
+
+void launch_survivors(const FusedGeom& G, const float* viewdirs, int64_t n_rays, int cap,
+                      const void* s4, const void* g4, const int* stats, const int64_t* cnt,
+                      const int64_t* off_incl, int64_t max_rows, void* P4, void* G4, int* rid,
+                      uint32_t* pages, hipStream_t st) {
+  k_survivors<<<(unsigned)cdiv(n_rays, 16), 256, 0, st>>>(
+      G, viewdirs, n_rays, cap, (const float4*)s4, (const float4*)g4, stats, cnt, off_incl,
+      max_rows, (float4*)P4, (float4*)G4, rid, pages);
+}
+
+// rgbnet rows X = [k0 (C) | normal (3) | view PE (3 + 6 nf) | 0 pad], 64 of the survivors a
+// workgroup and pass: k0 with a lane per row and four channels (or channel), the embedding
+// once for each ray among them (their rows are neighbours) with a lane per sine and cosine,
+// then the columns past C with sixteen lanes a row.
 // normal = grad / (|grad| + 1e-5) (lib/voxurf_fine.py:766 with the 1e-5 of :810);
 // view PE = [v, sin(v_i f_j), cos(v_i f_j)] with f_j = 2^j (lib/voxurf_fine.py:694-695).
-__global__ void __launch_bounds__(256) k_fused_gather(
-    FusedGeom G, const float* __restrict__ viewdirs, int64_t n_rays, int cap, int n_freq,
-    const float4* __restrict__ s4, const float4* __restrict__ g4, const int* __restrict__ stats,
-    const int64_t* __restrict__ cnt, const int64_t* __restrict__ off_incl, int xstride,
-    int64_t max_rows, float* __restrict__ X, float4* __restrict__ P4, float4* __restrict__ G4,
-    int* __restrict__ rid, uint32_t* __restrict__ pages) {
-  const int lane = threadIdx.x & 63, grp = lane >> 4, cl = lane & 15;
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
-  const int C = G.gk.C;
-  const int npe = 3 + 6 * n_freq;
+constexpr int kRowTile = 64;
+
+__global__ void __launch_bounds__(256) k_fused_rows(
+    FusedGeom G, const float* __restrict__ viewdirs, int64_t n_rays, int n_freq,
+    const int64_t* __restrict__ off_incl, int xstride, int64_t max_rows, float* __restrict__ X,
+    const float4* __restrict__ P4, const float4* __restrict__ G4, const int* __restrict__ rid) {
+  __shared__ float4 pos[kRowTile], nrml[kRowTile];  // nrml.w: the slot of the row's ray
+  __shared__ int ray[kRowTile];                     // [slot]
+  __shared__ int n_slots;
+  __shared__ float4 tail[kRowTile][16];             // [slot]: embeddings at column - (C & ~3)
+  const int tid = threadIdx.x;
+  const int C = G.gk.C, c0 = C & ~3;
+  const int npe = 3 + 6 * n_freq, half = 3 * n_freq;
   // channels innermost with 16-byte aligned corner rows: four channels per load
   const bool vec4 = G.gk.sc == 1 && (C & 3) == 0 && ((G.gk.sx | G.gk.sy | G.gk.sz) & 3) == 0 &&
                     (reinterpret_cast<uintptr_t>(G.k0) & 15) == 0;
-  for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); r < n_rays;
-       r += waves) {
-    const int64_t c = cnt[r];
-    if (c == 0) continue;
-    const int c1 = stats[3 * r + 1];
-    const int64_t o = off_incl[r] - c;
-    if (o >= max_rows && !pages) continue;  // past the output capacity (rows are not written)
-    const float* vd = viewdirs + 3 * r;
-    // view PE values of this lane's four columns (zero outside the PE block)
-    float pev[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int idx = 4 * cl + e - C - 3;
-      float v = 0.f;
-      if (idx >= 0 && idx < 3) {
-        v = vd[idx];
-      } else if (idx >= 3 && idx < npe) {
-        const int half = 3 * n_freq;
-        const int q = (idx - 3) % half;  // (component, freq) in component-major order
+  const int64_t total = off_incl[n_rays - 1];
+  const int64_t rows = total < max_rows ? total : max_rows;
+  for (int64_t row0 = blockIdx.x * (int64_t)kRowTile; row0 < rows; row0 += gridDim.x * (int64_t)kRowTile) {
+    const int m = (int)(rows - row0 < kRowTile ? rows - row0 : kRowTile);
+    if (tid < kRowTile) {
+      const int64_t j = row0 + (tid < m ? tid : m - 1);
+      const float4 a = P4[j], b = G4[j];
+      const int rr = rid[j];
+      const int before = __shfl_up(rr, 1, 64);
+      const uint64_t heads = __ballot(tid == 0 || rr != before);
+      const int slot = __popcll(heads & (lanemask_lt(tid) | (1ull << tid))) - 1;
+      const float nrm = sqrtf(b.x * b.x + b.y * b.y + b.z * b.z) + 1e-5f;
+      pos[tid] = a;
+      nrml[tid] = make_float4(b.x / nrm, b.y / nrm, b.z / nrm, __int_as_float(slot));
+      if (heads >> tid & 1) ray[slot] = min(max(rr, 0), (int)n_rays - 1);
+      if (tid == 0) n_slots = __popcll(heads);
+    }
+    __syncthreads();
+    const int nch = vec4 ? C >> 2 : C;
+    for (int i = tid; i < m * nch; i += 256) {
+      const int row = (int)((unsigned)i / (unsigned)nch), ch = i - row * nch;
+      const float4 q = pos[row];
+      Tri<float> t;
+      t.init(world_to_index(q.x, G.mn[0], G.mx[0] - G.mn[0], G.gk.X),
+             world_to_index(q.y, G.mn[1], G.mx[1] - G.mn[1], G.gk.Y),
+             world_to_index(q.z, G.mn[2], G.mx[2] - G.mn[2], G.gk.Z));
+      float* x = X + (row0 + row) * xstride;
+      if (vec4) *reinterpret_cast<float4*>(x + 4 * ch) = tri_gather4(G.k0, G.gk, t, 4 * ch);
+      else x[ch] = tri_gather(G.k0, G.gk, t, ch);
+    }
+    const int npt = half + 3, nt = n_slots * npt;
+    for (int i = 255 - tid; i < nt; i += 256) {
+      const int slot = (int)((unsigned)i / (unsigned)npt), k = i - slot * npt;
+      const float* vd = viewdirs + 3 * (int64_t)ray[slot];
+      float* pe = reinterpret_cast<float*>(tail[slot]) + (C + 3 - c0);
+      if (k < 3) {
+        pe[k] = vd[k];
+      } else {
+        const int q = k - 3;  // (component, freq) in component-major order
         const int comp = q / n_freq, f = q % n_freq;
         const float arg = vd[comp] * (float)(1 << f);
-        v = (idx - 3 < half) ? sinf(arg) : cosf(arg);
+        pe[3 + q] = sinf(arg);
+        pe[3 + half + q] = cosf(arg);
       }
-      pev[e] = v;
     }
-    int64_t ks = 0;
-    for (int base = 0; base < c1; base += 64) {
-      const int k = base + lane;
-      float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-      bool surv = false;
-      float w = 0.f;
-      if (k < c1) {
-        a = s4[r * cap + k];
-        b = g4[r * cap + k];
-        SlotSample ss;
-        load_slot(G, vd, a, b, ss);
-        w = ss.w;
-        surv = ss.w > G.thres;
-      }
-      const uint64_t sm = __ballot(surv);
-      // rows past the forward's survivor count are never written (they cannot occur:
-      // the recomputed weights are the forward's)
-      const int64_t room = c - ks;
-      const int rank = __popcll(sm & lanemask_lt(lane));
-      if (surv && rank < room && o + ks + rank < max_rows) {
-        const int64_t j = o + ks + rank;
-        P4[j] = make_float4(a.x, a.y, a.z, w);
-        G4[j] = b;
-        rid[j] = (int)r;
-      }
-      const int ns = (int)(__popcll(sm) < room ? __popcll(sm) : room);
-      for (int i = 0; i < ns; i += 4) {
-        const int kk = i + grp;
-        const bool on = kk < ns;
-        const int src = kth_set_bit(sm, on ? kk : 0);
-        const float qx = __shfl(a.x, src, 64), qy = __shfl(a.y, src, 64), qz = __shfl(a.z, src, 64);
-        const float gx = __shfl(b.x, src, 64), gy = __shfl(b.y, src, 64), gz = __shfl(b.z, src, 64);
-        if (on) {
-          Tri<float> t;
-          t.init(world_to_index(qx, G.mn[0], G.mx[0] - G.mn[0], G.gk.X),
-                 world_to_index(qy, G.mn[1], G.mx[1] - G.mn[1], G.gk.Y),
-                 world_to_index(qz, G.mn[2], G.mx[2] - G.mn[2], G.gk.Z));
-          if (pages && cl < 8) mark_corner_pages(pages, G.gk, t, cl);
-          if (4 * cl < xstride && o + ks + kk < max_rows) {
-            const float nrm = sqrtf(gx * gx + gy * gy + gz * gz) + 1e-5f;
-            float v[4];
-            if (vec4 && 4 * cl + 3 < C) {
-              const float4 f = tri_gather4(G.k0, G.gk, t, 4 * cl);
-              v[0] = f.x;
-              v[1] = f.y;
-              v[2] = f.z;
-              v[3] = f.w;
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const int col = 4 * cl + e;
-                float x = pev[e];
-                if (col < C) {
-                  x = tri_gather(G.k0, G.gk, t, col);
-                } else if (col < C + 3) {
-                  const float comp = (col == C) ? gx : (col == C + 1 ? gy : gz);
-                  x = comp / nrm;
-                }
-                v[e] = x;
-              }
-            }
-            *reinterpret_cast<float4*>(X + (o + ks + kk) * xstride + 4 * cl) =
-                make_float4(v[0], v[1], v[2], v[3]);
-          }
+    __syncthreads();
+    // the columns past C
+    for (int row = tid >> 4; row < m; row += 16) {
+      const float4 n4 = nrml[row];
+      const float4* tl = tail[__float_as_int(n4.w)];
+      float* x = X + (row0 + row) * xstride;
+      auto value = [&](int col, float pe) {
+        if (col < C + 3) return col == C ? n4.x : (col == C + 1 ? n4.y : n4.z);
+        return col < C + 3 + npe ? pe : 0.f;
+      };
+      if ((C & 3) == 0) {
+        const int col = C + 4 * (tid & 15);
+        if (col < xstride) {
+          const float4 pe = tl[tid & 15];
+          *reinterpret_cast<float4*>(x + col) = make_float4(
+              value(col, pe.x), value(col + 1, pe.y), value(col + 2, pe.z), value(col + 3, pe.w));
         }
+      } else {
+        for (int col = C + (tid & 15); col < xstride; col += 16)
+          x[col] = value(col, reinterpret_cast<const float*>(tl)[col - c0]);
       }
-      ks += ns;
-      if (ks >= c) break;
     }
+    __syncthreads();
   }
 }
 
@@ -1168,9 +1214,14 @@ int vx_fused_fine_gather(const float* k0, const int64_t* k0_geom, const int64_t*
   VX_CHECK_ARG(cap >= 1, "fused_fine_gather: cap < 1");
   if (int st = check_corner_pages("fused_fine_gather", G, k0_pages)) return st;
   if (n_rays == 0) return VX_OK;
-  k_fused_gather<<<grid_for(n_rays, 4, 1 << 16), 256, 0, (hipStream_t)stream>>>(
-      G, viewdirs, n_rays, cap, n_freq, (const float4*)s4, (const float4*)g4, stats, cnt,
-      off_incl, xstride, max_rows, X, (float4*)P4, (float4*)G4, rid, k0_pages);
+  hipStream_t st = (hipStream_t)stream;
+  launch_survivors(G, viewdirs, n_rays, cap, s4, g4, stats, cnt, off_incl, max_rows, P4, G4, rid,
+                   k0_pages, st);
+  // max_rows may be a capacity far past the survivors: a few passes for a full one
+  if (max_rows > 0)
+    k_fused_rows<<<grid_for(max_rows, kRowTile, 1 << 12), 256, 0, st>>>(
+        G, viewdirs, n_rays, n_freq, off_incl, xstride, max_rows, X, (const float4*)P4,
+        (const float4*)G4, rid);
   return launch_status("fused_fine_gather");
 }
 

@@ -6,10 +6,8 @@
 // compositing; rgb_marched0 (sigmoid(rgb_logit) composited) feeds the second MSE term.
 //
 // The per-ray forward, the survivor scan and the SDF backward are the plain fine step's
-// (fused.hip).  Here: the row builder (one wavefront per ray, four survivor rows per
-// pass, sixteen lanes per row; the 2 x 3 x nd displaced SDF samples of sample_sdfs are
-// spread over the row's lanes, two per lane, and shuffled to the lanes that own their
-// columns), the compositing with both colour terms, the loss and the entropy of the last
+// (fused.hip).  Here: the row builder (tiles of 32 survivor rows put together in LDS, a lane
+// per displaced SDF sample of sample_sdfs, sine and cosine), the compositing with both colour terms, the loss and the entropy of the last
 // ray, and the adjoint of the rows (k0 scatter, the raw-gradient and centre-SDF
 // adjoints handed to the SDF backward, and the displaced-sample scatter of sample_sdfs).
 // Every per-value formula is the drop-in ops' own (voxel.h), so the rows equal the
@@ -28,18 +26,6 @@ struct VoxurfRowDesc {
   int x_view, x_sdf, x_feat, x_grad, x_end;
   int k_pos, k_view, k_grad, k_logit, k_end;
 };
-
-// [x, sin(x_c 2^f) (component-major), cos(...)] element idx of an embedding with nf
-// frequencies (lib/voxurf_fine.py:694-698).
-__device__ __forceinline__ float pe_val(int idx, const float x[3], int nf) {
-#pragma clang fp contract(off)
-  if (idx < 3) return x[idx];
-  const int half = 3 * nf;
-  const int q = (idx - 3) % half;
-  const int comp = q / nf, f = q % nf;
-  const float arg = x[comp] * (float)(1 << f);
-  return (idx - 3 < half) ? sinf(arg) : cosf(arg);
-}
 
 // One lane's share of sample_sdfs for one row: lane l < 3 nd takes axis a = l / nd and
 // displacement j = l % nd, i.e. the samples at -d and +d along a (zyx index space) and
@@ -69,135 +55,143 @@ __device__ __forceinline__ void hier_lane(const FusedGeom& G, const VoxurfRowDes
   h.r = ((h.fp - h.fm) / h.df) / G.voxel_size;
 }
 
-// Rows of the survivors.  Per ray: one wavefront walks its walk-range slots 64 at a time,
-// keeps the survivors (w > thres) at rows off[r] .. off[r] + cnt[r] - 1 (P4, G4, rid as
-// the plain gather), and fills X and XK four rows per pass.  XK's logit columns are
-// left zero (vx_voxurf_logit_cols fills them after rgbnet's forward).
-__global__ void __launch_bounds__(256) k_voxurf_gather(
-    FusedGeom G, VoxurfRowDesc D, const float* __restrict__ viewdirs, int64_t n_rays, int cap,
-    const float4* __restrict__ s4, const float4* __restrict__ g4, const int* __restrict__ stats,
-    const int64_t* __restrict__ cnt, const int64_t* __restrict__ off_incl, int64_t max_rows,
-    float* __restrict__ X, float* __restrict__ XK, float4* __restrict__ P4,
-    float4* __restrict__ G4, int* __restrict__ rid) {
-  const int lane = threadIdx.x & 63, grp = lane >> 4, cl = lane & 15;
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
-  const int C = G.gk.C;
-  for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); r < n_rays;
-       r += waves) {
-    const int64_t c = cnt[r];
-    if (c == 0) continue;
-    const int c1 = stats[3 * r + 1];
-    const int64_t o = off_incl[r] - c;
-    if (o >= max_rows) continue;  // past the output capacity (rows are not written)
-    const float vd[3] = {viewdirs[3 * r], viewdirs[3 * r + 1], viewdirs[3 * r + 2]};
-    int64_t ks = 0;
-    for (int base = 0; base < c1; base += 64) {
-      const int k = base + lane;
-      float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-      bool surv = false;
-      if (k < c1) {
-        a = s4[r * cap + k];
-        b = g4[r * cap + k];
-        SlotSample ss;
-        load_slot(G, vd, a, b, ss);
-        surv = ss.w > G.thres;
-        a.w = ss.w;
-      }
-      const uint64_t sm = __ballot(surv);
-      const int64_t room = c - ks;
-      const int rank = __popcll(sm & lanemask_lt(lane));
-      if (surv && rank < room && o + ks + rank < max_rows) {
-        const int64_t j = o + ks + rank;
-        P4[j] = a;
-        G4[j] = b;
-        rid[j] = (int)r;
-      }
-      const int ns = (int)(__popcll(sm) < room ? __popcll(sm) : room);
-      for (int i = 0; i < ns; i += 4) {
-        const int kk = i + grp;
-        const bool on = kk < ns;
-        const int src = kth_set_bit(sm, on ? kk : 0);
-        float q[3] = {__shfl(a.x, src, 64), __shfl(a.y, src, 64), __shfl(a.z, src, 64)};
-        const float gx = __shfl(b.x, src, 64), gy = __shfl(b.y, src, 64),
-                    gz = __shfl(b.z, src, 64), sd = __shfl(b.w, src, 64);
-        const int64_t row = o + ks + kk;
-        const bool write = on && row < max_rows;
-        // this lane's share of the displaced samples, then the normalisation over the
-        // three axes of each displacement (lanes j, nd + j, 2 nd + j of the row)
-        HierLane h;
-        hier_lane(G, D, q, on ? cl : 64, h);
-        const int gbase = grp * 16;
-        const float r0 = __shfl(h.r, gbase + h.j, 64);
-        const float r1 = __shfl(h.r, gbase + D.nd + h.j, 64);
-        const float r2 = __shfl(h.r, gbase + 2 * D.nd + h.j, 64);
-        float grn;
-        {
+// Rows X and XK of the survivors, 32 a workgroup and pass, put together in LDS (dynamic: the
+// two tiles of rows) and written out in one run each.  Every value is a lane's own task: the
+// 6 nd displaced samples of a row (minus and plus in neighbouring lanes), the sines and
+// cosines (once for both rows), four channels of k0.  A wavefront per ray with sixteen lanes a
+// row before, twelve of them taking two samples in turn and each working out its columns'
+// embeddings with runtime divisions, was bound by those instructions: 491 us for 29,000 rows
+// of an 8192-ray chunk, 50 so.  XK's logit columns are left zero (vx_voxurf_logit_cols
+// fills them after rgbnet's forward).
+constexpr int kVxRowTile = 32;
+
+__global__ void __launch_bounds__(256) k_voxurf_rows(
+    FusedGeom G, VoxurfRowDesc D, const float* __restrict__ viewdirs, int64_t n_rays,
+    const int64_t* __restrict__ off_incl, int64_t max_rows, float* __restrict__ X,
+    float* __restrict__ XK, const float4* __restrict__ P4, const float4* __restrict__ G4,
+    const int* __restrict__ rid) {
+  extern __shared__ float4 tiles[];
+  __shared__ float raw[kVxRowTile][3 * kVxMaxDisp];  // unnormalised gradients [axis][displacement]
+  __shared__ float ind[kVxRowTile][4], unit[kVxRowTile][4], dir[kVxRowTile][4];
+  __shared__ float4 pos[kVxRowTile], grad[kVxRowTile];
+  float* xr = reinterpret_cast<float*>(tiles);
+  float* kr = xr + kVxRowTile * D.xstride;
+  const int tid = threadIdx.x, C = G.gk.C, nd = D.nd;
+  const bool vec4 = G.gk.sc == 1 && (C & 3) == 0 && ((G.gk.sx | G.gk.sy | G.gk.sz) & 3) == 0 &&
+                    (reinterpret_cast<uintptr_t>(G.k0) & 15) == 0;
+  const int64_t total = off_incl[n_rays - 1];
+  const int64_t rows = total < max_rows ? total : max_rows;
+  for (int64_t row0 = blockIdx.x * (int64_t)kVxRowTile; row0 < rows;
+       row0 += gridDim.x * (int64_t)kVxRowTile) {
+    const int m = (int)(rows - row0 < kVxRowTile ? rows - row0 : kVxRowTile);
+    for (int i = tid; i < kVxRowTile * (D.xstride + D.kstride) / 4; i += 256)
+      tiles[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (tid < m) {
 #pragma clang fp contract(off)
-          const float nrm = sqrtf(r0 * r0 + r1 * r1 + r2 * r2) + 1e-5f;
-          grn = h.r / nrm;
-        }
-        // normalised point for the xyz PE: (p - min) / (max - min)
-        float u[3];
-        {
-#pragma clang fp contract(off)
-          for (int e = 0; e < 3; ++e) u[e] = (q[e] - G.mn[e]) / (G.mx[e] - G.mn[e]);
-        }
-        Tri<float> t;
-        t.init(world_to_index(q[0], G.mn[0], G.mx[0] - G.mn[0], G.gk.X),
-               world_to_index(q[1], G.mn[1], G.mx[1] - G.mn[1], G.gk.Y),
-               world_to_index(q[2], G.mn[2], G.mx[2] - G.mn[2], G.gk.Z));
-        // rgbnet row: float4 groups cl and cl + 16
-#pragma unroll
-        for (int gi = 0; gi < 2; ++gi) {
-          const int g0 = 4 * (cl + 16 * gi);
-          float v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int col = g0 + e;
-            // displaced-sample columns: the computing lane and which of its values
-            int hl = 0, sel = 0;  // sel 1: f-, 2: f+, 3: normalised gradient
-            if (col >= D.x_feat && col < D.x_grad) {
-              const int f = col - D.x_feat, oo = f / D.nd, jj = f % D.nd;
-              hl = (oo >> 1) * D.nd + jj;
-              sel = (oo & 1) ? 2 : 1;
-            } else if (col >= D.x_grad && col < D.x_end) {
-              hl = col - D.x_grad;
-              sel = 3;
-            }
-            const float vm = __shfl(h.fm, gbase + hl, 64);
-            const float vp = __shfl(h.fp, gbase + hl, 64);
-            const float vg = __shfl(grn, gbase + hl, 64);
-            float x = 0.f;
-            if (sel == 1) x = vm;
-            else if (sel == 2) x = vp;
-            else if (sel == 3) x = vg;
-            else if (col < D.x_view) x = pe_val(col, u, D.pos_pe);
-            else if (col < D.x_sdf) x = pe_val(col - D.x_view, vd, D.view_pe);
-            else if (col == D.x_sdf) x = sd;
-            v[e] = x;
-          }
-          if (write && g0 < D.xstride)
-            *reinterpret_cast<float4*>(X + row * D.xstride + g0) = make_float4(v[0], v[1], v[2], v[3]);
-        }
-        // k_rgbnet row: float4 group cl
-        if (write && 4 * cl < D.kstride) {
-          float v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int col = 4 * cl + e;
-            float x = 0.f;
-            if (col < C) x = tri_gather(G.k0, G.gk, t, col);
-            else if (col < D.k_view) x = pe_val(col - D.k_pos, u, D.pos_pe);
-            else if (col < D.k_grad) x = pe_val(col - D.k_view, vd, D.k_view_pe);
-            else if (col < D.k_logit) x = (col == D.k_grad) ? gx : (col == D.k_grad + 1 ? gy : gz);
-            v[e] = x;
-          }
-          *reinterpret_cast<float4*>(XK + row * D.kstride + 4 * cl) = make_float4(v[0], v[1], v[2], v[3]);
-        }
+      const float4 a = P4[row0 + tid];
+      const int64_t r = min(max(rid[row0 + tid], 0), (int)n_rays - 1);
+      const float q[3] = {a.x, a.y, a.z};
+      float id[3];
+      zyx_index(q, G.mn, G.mx, G.gs, id);
+      for (int e = 0; e < 3; ++e) {
+        ind[tid][e] = id[e];
+        unit[tid][e] = (q[e] - G.mn[e]) / (G.mx[e] - G.mn[e]);  // for the xyz PE
+        dir[tid][e] = viewdirs[3 * r + e];
       }
-      ks += ns;
-      if (ks >= c) break;
+      pos[tid] = a;
+      grad[tid] = G4[row0 + tid];
     }
+    __syncthreads();
+    // sample_sdfs: the value at -d (even tasks) and +d (odd) along each axis, and the
+    // gradient component (f+ - f-) / diff / voxel_size, as k_sdfs_fwd
+    const int n6 = 6 * nd;
+    for (int i = tid; i < m * n6; i += 256) {
+#pragma clang fp contract(off)
+      const int row = (int)((unsigned)i / (unsigned)n6), t = i - row * n6;
+      const int sgn = t & 1, hl = t >> 1, a = (int)((unsigned)hl / (unsigned)nd), j = hl - a * nd;
+      const float id[3] = {ind[row][0], ind[row][1], ind[row][2]};
+      const float d = D.disp[j];
+      float cl;
+      const float f = sample_displaced(G.sdf, G.gs, id, a, sgn ? d : -d, cl);
+      xr[row * D.xstride + D.x_feat + (2 * a + sgn) * nd + j] = f;
+      const float fm = __shfl_xor(f, 1, 64);
+      if (sgn) raw[row][hl] = ((f - fm) / clamped_diff(id, a, d, G.gs)) / G.voxel_size;
+    }
+    const int np3 = 3 * D.pos_pe;
+    for (int i = tid; i < m * np3; i += 256) {
+#pragma clang fp contract(off)
+      const int row = (int)((unsigned)i / (unsigned)np3), t = i - row * np3;
+      const int comp = (int)((unsigned)t / (unsigned)D.pos_pe), f = t - comp * D.pos_pe;
+      const float arg = unit[row][comp] * (float)(1 << f);
+      const float sn = sinf(arg), cs = cosf(arg);
+      float* x = xr + row * D.xstride + 3 + t;
+      float* k = kr + row * D.kstride + D.k_pos + 3 + t;
+      x[0] = sn;
+      x[np3] = cs;
+      k[0] = sn;
+      k[np3] = cs;
+    }
+    const int nv = max(D.view_pe, D.k_view_pe), nv3 = 3 * nv;
+    for (int i = tid; i < m * nv3; i += 256) {
+#pragma clang fp contract(off)
+      const int row = (int)((unsigned)i / (unsigned)nv3), t = i - row * nv3;
+      const int comp = (int)((unsigned)t / (unsigned)nv), f = t - comp * nv;
+      const float arg = dir[row][comp] * (float)(1 << f);
+      const float sn = sinf(arg), cs = cosf(arg);
+      if (f < D.view_pe) {
+        float* x = xr + row * D.xstride + D.x_view + 3 + comp * D.view_pe + f;
+        x[0] = sn;
+        x[3 * D.view_pe] = cs;
+      }
+      if (f < D.k_view_pe) {
+        float* k = kr + row * D.kstride + D.k_view + 3 + comp * D.k_view_pe + f;
+        k[0] = sn;
+        k[3 * D.k_view_pe] = cs;
+      }
+    }
+    const int nch = vec4 ? C >> 2 : C;
+    for (int i = 255 - tid; i < m * nch; i += 256) {
+      const int row = (int)((unsigned)i / (unsigned)nch), ch = i - row * nch;
+      const float4 q = pos[row];
+      Tri<float> t;
+      t.init(world_to_index(q.x, G.mn[0], G.mx[0] - G.mn[0], G.gk.X),
+             world_to_index(q.y, G.mn[1], G.mx[1] - G.mn[1], G.gk.Y),
+             world_to_index(q.z, G.mn[2], G.mx[2] - G.mn[2], G.gk.Z));
+      float* k = kr + row * D.kstride;
+      if (vec4) *reinterpret_cast<float4*>(k + 4 * ch) = tri_gather4(G.k0, G.gk, t, 4 * ch);
+      else k[ch] = tri_gather(G.k0, G.gk, t, ch);
+    }
+    for (int i = tid; i < m * 4; i += 256) {
+      const int row = i >> 2, e = i & 3;
+      float* x = xr + row * D.xstride;
+      float* k = kr + row * D.kstride;
+      const float4 g = grad[row];
+      if (e < 3) {
+        x[e] = k[D.k_pos + e] = unit[row][e];
+        x[D.x_view + e] = k[D.k_view + e] = dir[row][e];
+        k[D.k_grad + e] = e == 0 ? g.x : (e == 1 ? g.y : g.z);
+      } else {
+        x[D.x_sdf] = g.w;
+      }
+    }
+    __syncthreads();
+    // normalised over the three axes of each displacement
+    for (int i = tid; i < m * nd; i += 256) {
+#pragma clang fp contract(off)
+      const int row = (int)((unsigned)i / (unsigned)nd), j = i - row * nd;
+      const float r0 = raw[row][j], r1 = raw[row][nd + j], r2 = raw[row][2 * nd + j];
+      const float nrm = sqrtf(r0 * r0 + r1 * r1 + r2 * r2) + 1e-5f;
+      float* x = xr + row * D.xstride + D.x_grad + j;
+      x[0] = r0 / nrm;
+      x[nd] = r1 / nrm;
+      x[2 * nd] = r2 / nrm;
+    }
+    __syncthreads();
+    float4* xo = reinterpret_cast<float4*>(X + row0 * D.xstride);
+    float4* ko = reinterpret_cast<float4*>(XK + row0 * D.kstride);
+    for (int i = tid; i < m * D.xstride / 4; i += 256) xo[i] = tiles[i];
+    for (int i = tid; i < m * D.kstride / 4; i += 256) ko[i] = reinterpret_cast<float4*>(kr)[i];
+    __syncthreads();
   }
 }
 
@@ -483,9 +477,13 @@ int vx_voxurf_gather(const float* sdf, const int64_t* sdf_geom, const float* k0,
   if (int st = voxurf_desc(D, G, row_cfg, disp)) return st;
   VX_CHECK_ARG(cap >= 1 && n_rays >= 0, "voxurf_gather: bad sizes");
   if (n_rays == 0) return VX_OK;
-  k_voxurf_gather<<<grid_for(n_rays, 4, 1 << 16), 256, 0, (hipStream_t)stream>>>(
-      G, D, viewdirs, n_rays, cap, (const float4*)s4, (const float4*)g4, stats, cnt, off_incl,
-      max_rows, X, XK, (float4*)P4, (float4*)G4, rid);
+  hipStream_t st = (hipStream_t)stream;
+  launch_survivors(G, viewdirs, n_rays, cap, s4, g4, stats, cnt, off_incl, max_rows, P4, G4, rid,
+                   nullptr, st);
+  if (max_rows > 0)
+    k_voxurf_rows<<<grid_for(max_rows, kVxRowTile, 1 << 12), 256,
+                    kVxRowTile * (D.xstride + D.kstride) * 4, st>>>(
+        G, D, viewdirs, n_rays, off_incl, max_rows, X, XK, (const float4*)P4, (const float4*)G4, rid);
   return launch_status("voxurf_gather");
 }
 
