@@ -24,27 +24,52 @@ struct FusedGeom {
   const float4* skip;
   int skx, sky, skz;
   float skip_xmin;
+  float skip_scale[3];  // voxels per world unit
 };
 
 constexpr int kSkipShift = 3;  // empty-space bricks of 8^3 cells
 
-// True when the in-box sample at q provably has NeuS alpha <= thres, so that it takes no
-// part in the walk (lib/voxurf_fine.py keeps alpha > thres only): with c = sigmoid(prev
-// inv_s) and n = sigmoid(next inv_s), alpha = (c - n + 1e-5) / (c + 1e-5), and
-// next = sdf - |h| <= prev, |h| = |cos| dist / 2 <= |viewdir| |grad| dist / 2; once
-// next inv_s >= x_min = ln(1 / (thres - 2e-5)) + 1, c - n <= e^-x_min (plus float
-// rounding) and alpha stays below thres.  hfac = |viewdir| dist / 2 of the ray (with a
-// margin); the brick's bounds hold for every voxel of the 7-point stencil of any sample
-// whose cell lies in it.
-__device__ __forceinline__ bool skip_sample(const FusedGeom& G, const float q[3], float hfac) {
-  const float fx = world_to_index(q[0], G.mn[0], G.mx[0] - G.mn[0], G.gs.X);
-  const float fy = world_to_index(q[1], G.mn[1], G.mx[1] - G.mn[1], G.gs.Y);
-  const float fz = world_to_index(q[2], G.mn[2], G.mx[2] - G.mn[2], G.gs.Z);
-  const int bx = min(max(sat_f2i(floorf(fx)) >> kSkipShift, 0), G.skx - 1);
-  const int by = min(max(sat_f2i(floorf(fy)) >> kSkipShift, 0), G.sky - 1);
-  const int bz = min(max(sat_f2i(floorf(fz)) >> kSkipShift, 0), G.skz - 1);
+// Empty space along a ray, eight steps at a time.  A sample provably has NeuS alpha <= thres,
+// so that it takes no part in the walk (lib/voxurf_fine.py keeps alpha > thres only), when with
+// c = sigmoid(prev inv_s), n = sigmoid(next inv_s), alpha = (c - n + 1e-5) / (c + 1e-5) and
+// next = sdf - |h| <= prev, |h| = |cos| dist / 2 <= |viewdir| |grad| dist / 2, next inv_s >=
+// x_min = ln(1 / (thres - 2e-5)) + 1: c - n <= e^-x_min (plus float rounding) and alpha stays
+// below thres.
+//
+// A brick's bounds on the SDF and its gradient hold over the voxels from 8 below its first
+// cell to 8 above its last, and a sample reads from 2 below its cell to 3 above it: they hold
+// for every sample within five cells of the brick.  So the brick of the fifth of eight steps
+// speaks for all eight while four steps are no longer than 4.5 voxels along any axis (the
+// index of that step need not be exact either).
+constexpr int kSkipGroup = 8;
+struct SkipRay {
+  float b[3], a[3];  // index of step s along axis k: b + a s
+  float hfac;        // |viewdir| dist / 2 (with a margin)
+  bool on, eights;   // empty space is known; eight steps at a time
+};
+
+__device__ __forceinline__ void skip_ray(const FusedGeom& G, const float start[3],
+                                         const float dir[3], const float* vd, SkipRay& k) {
+  k.on = k.eights = false;
+  if (!G.skip) return;
+  k.on = true;
+  k.hfac = sqrtf(vd[0] * vd[0] + vd[1] * vd[1] + vd[2] * vd[2]) * G.stepdist * 0.5f * (1.f + 1e-4f);
+  float longest = 0.f;
+  for (int e = 0; e < 3; ++e) {
+    k.b[e] = (start[e] - G.mn[e]) * G.skip_scale[e];
+    k.a[e] = dir[e] * G.stepdist * G.skip_scale[e];
+    longest = fmaxf(longest, fabsf(k.a[e]));
+  }
+  k.eights = longest * (kSkipGroup / 2) <= 4.5f;
+}
+
+__device__ __forceinline__ bool skip_at(const FusedGeom& G, const SkipRay& k, int64_t step) {
+  const float s = (float)(int)step;
+  const int bx = min(max(sat_f2i(floorf(fmaf(k.a[0], s, k.b[0]))) >> kSkipShift, 0), G.skx - 1);
+  const int by = min(max(sat_f2i(floorf(fmaf(k.a[1], s, k.b[1]))) >> kSkipShift, 0), G.sky - 1);
+  const int bz = min(max(sat_f2i(floorf(fmaf(k.a[2], s, k.b[2]))) >> kSkipShift, 0), G.skz - 1);
   const float4 b = G.skip[((int64_t)bx * G.sky + by) * G.skz + bz];
-  return (b.x * (1.f - 1e-6f) - hfac * b.y) * G.inv_s >= G.skip_xmin;
+  return (b.x * (1.f - 1e-6f) - k.hfac * b.y) * G.inv_s >= G.skip_xmin;
 }
 
 // MaskCache.forward for one point (lib/voxurf_fine.py:930-942), as vx_maskcache_alpha: the
@@ -162,6 +187,8 @@ static inline void fused_skip(FusedGeom& G, const void* bounds) {
   G.sky = (G.gs.Y + (1 << kSkipShift) - 1) >> kSkipShift;
   G.skz = (G.gs.Z + (1 << kSkipShift) - 1) >> kSkipShift;
   G.skip_xmin = logf(1.f / (G.thres - 2e-5f)) + 1.f;
+  const int size[3] = {G.gs.X, G.gs.Y, G.gs.Z};
+  for (int e = 0; e < 3; ++e) G.skip_scale[e] = (float)(size[e] - 1) / (G.mx[e] - G.mn[e]);
 }
 
 // mc_params = {act_shift, voxel_size_ratio, thres, nearest, xyz_min[3], xyz_max[3]}

@@ -385,20 +385,61 @@ __device__ __forceinline__ void sdf7(const T* __restrict__ grid, const GridDesc&
   // 8 corner values are selected from them (the same values, weights and sums as 56
   // separate loads); otherwise every cell loads its own corners.
   int dd[6];
-  bool shared = true;
+  bool shared = true, shifted = true;
 #pragma unroll
   for (int i = 1; i < 7; ++i) {
     const int c = 2 - (i - 1) / 2, s = (i - 1) % 2 ? 1 : -1;  // world axis, side
     const int d[3] = {t[i].x0 - t[0].x0, t[i].y0 - t[0].y0, t[i].z0 - t[0].z0};
     dd[i - 1] = d[c];
     shared = shared && d[(c + 1) % 3] == 0 && d[(c + 2) % 3] == 0 && (d[c] == 0 || d[c] == s);
+    shifted = shifted && d[c] == s;
   }
   if (shared_out) *shared_out = shared;
   T f[7];  // the seven lookups: centre, then -/+ along z, y, x of the zyx index
   // element offsets in 32 bits (the grid is below 2^31 elements; uniform)
   const bool idx32 = (int64_t)(g.X - 1) * g.sx + (int64_t)(g.Y - 1) * g.sy +
                          (int64_t)(g.Z - 1) * g.sz < ((int64_t)1 << 31);
-  if (idx32 && __all(shared)) {
+  // Away from the faces nothing is clamped and every voxel is in the grid: the 32 voxels in
+  // twelve runs along z (four of 4, eight of 2), no selections.  (k_sdf_grad_fwd over the
+  // samples of 8192 coarse rays 100 -> 71 us: address arithmetic and cache accesses.)
+  const bool inner = shared && shifted && (unsigned)(t[0].x0 - 1) < (unsigned)max(g.X - 3, 0) &&
+                     (unsigned)(t[0].y0 - 1) < (unsigned)max(g.Y - 3, 0) &&
+                     (unsigned)(t[0].z0 - 1) < (unsigned)max(g.Z - 3, 0);
+  if (sizeof(T) == 4 && idx32 && g.sz == 1 && __all(inner)) {
+    typedef T run4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    typedef T run2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    const int sx = (int)g.sx, sy = (int)g.sy;
+    const int o = t[0].x0 * sx + t[0].y0 * sy + t[0].z0;
+    run4 mid[2][2];
+    run2 ox[2][2], oy[2][2];  // [side][the other of x, y]: one cell out along x, along y
+#pragma unroll
+    for (int dx = 0; dx < 2; ++dx)
+#pragma unroll
+      for (int dy = 0; dy < 2; ++dy)
+        mid[dx][dy] = *reinterpret_cast<const run4*>(grid + (o + dx * sx + dy * sy - 1));
+#pragma unroll
+    for (int side = 0; side < 2; ++side)
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        ox[side][d] = *reinterpret_cast<const run2*>(grid + (o + (side ? 2 : -1) * sx + d * sy));
+        oy[side][d] = *reinterpret_cast<const run2*>(grid + (o + d * sx + (side ? 2 : -1) * sy));
+      }
+    auto at = [&](int dx, int dy, int dz) {
+      if (dx == -1 || dx == 2) return ox[dx == 2][dy][dz];
+      if (dy == -1 || dy == 2) return oy[dy == 2][dx][dz];
+      return mid[dx][dy][dz + 1];
+    };
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+      const int c = 2 - (i - 1) / 2, s = i == 0 ? 0 : ((i - 1) % 2 ? 1 : -1);
+      T v[8];
+#pragma unroll
+      for (int b = 0; b < 8; ++b)
+        v[b] = at((b >> 2) + (c == 0 ? s : 0), ((b >> 1) & 1) + (c == 1 ? s : 0),
+                  (b & 1) + (c == 2 ? s : 0));
+      f[i] = tri_sum(t[i], v, 255u);
+    }
+  } else if (idx32 && __all(shared)) {
     // per axis, the clamped offsets and in-grid flags of lattice lines base-1 .. base+2
     int ox[4], oy[4], oz[4];
     unsigned vx = 0u, vy = 0u, vz = 0u;
