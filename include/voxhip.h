@@ -383,6 +383,15 @@ int vx_neus_alpha_bwd(int dtype, const void* viewdirs, const int64_t* ray_id, co
                       const void* gradient, int64_t n, double dist, double inv_s,
                       const void* galpha, void* gsdf, void* ggradient, void* stream);
 
+/* Row selection by a boolean mask [n] (one byte each; 1 <= n < 2^31): offsets
+ * [vx_select_blocks(n)] and total [1] (device) of the selected elements, then up to eight
+ * arrays (host arrays of device addresses, words: 32-bit words a row) copied under them:
+ * dst [total] = src[mask]; transpose = 1: dst [n] = src at the selected rows, zero elsewhere. */
+int64_t vx_select_blocks(int64_t n);
+int vx_select_count(const uint8_t* mask, int64_t n, int* offsets, int64_t* total, void* stream);
+int vx_select_rows(const uint8_t* mask, int64_t n, const int* offsets, int count,
+                   const int64_t* src, const int64_t* dst, const int* words, int transpose,
+                   void* stream);
 /* torch_scatter.segment_coo(src, index, out, reduce='sum') as called at
  * lib/voxurf_fine.py:753-777: out [n_out, C] += segment sums of src [n, C] over the
  * sorted index [n]. */

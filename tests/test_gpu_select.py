@@ -1,0 +1,51 @@
+"""Row selection of several arrays under one mask (vx_select_count, vx_select_rows) against
+x[mask]: the same bits and the same gradients, over lengths around the tiles of 4096, none, some
+and all rows, element types and row widths, strided and unaligned inputs, and the forms that
+are indexed instead."""
+import pytest
+import torch
+
+from voxurf_amd.functional import select_rows
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 257, 4095, 4096, 4097, 100003])
+@pytest.mark.parametrize("density", [0.0, 0.01, 0.5, 1.0])
+def test_equals_indexing(dev, n, density):
+    g = torch.Generator(device=dev).manual_seed(n)
+    r = lambda *s, dt=torch.float32: torch.randn(*s, generator=g, device=dev, dtype=dt)
+    base = torch.rand(n + 1, generator=g, device=dev) < density
+    ids = torch.randint(0, 1 << 40, (n,), generator=g, device=dev)
+    arrays = [r(n), r(n, 3), ids, r(n, 3, dt=torch.float64), r(3, n).T, r(n, 2, 5), r(2 * n)[::2],
+              ids.int()]
+    for mask in (base[:n].clone(), base[1:]):  # the second: not 16-byte aligned
+        xs = [a.detach().clone() if i not in (4, 6) else a.detach() for i, a in enumerate(arrays)]
+        for a in xs:
+            if a.is_floating_point() and a.dtype == torch.float32:
+                a.requires_grad_(True)
+        got, want = select_rows(mask, *xs), [a[mask] for a in xs]
+        for a, b in zip(got, want):
+            assert a.dtype == b.dtype and a.requires_grad == b.requires_grad and torch.equal(a, b)
+        gs = [torch.randn_like(b) for b in want if b.requires_grad]
+        leaves = [a for a in xs if a.requires_grad]
+        ga = torch.autograd.grad([a for a in got if a.requires_grad], leaves, gs)
+        gb = torch.autograd.grad([b for b in want if b.requires_grad], leaves, gs)
+        for a, b in zip(ga, gb):
+            assert a.shape == b.shape and torch.equal(a, b)
+
+
+def test_other_forms_are_indexed(dev):
+    mask = torch.tensor([True, False, True], device=dev)
+    b = torch.tensor([[True], [False], [True]], device=dev)         # one byte a row
+    h = torch.arange(3, device=dev, dtype=torch.float16)            # half a word
+    for a in (b, h, torch.zeros((3, 0), device=dev)):
+        assert torch.equal(select_rows(mask, a)[0], a[mask])
+    assert select_rows(mask[:0], torch.zeros(0, device=dev))[0].numel() == 0
+    # an unused output's gradient
+    x, y = (torch.ones(3, device=dev, requires_grad=True) for _ in range(2))
+    u, _ = select_rows(mask, x, y)
+    u.sum().backward()
+    assert torch.equal(x.grad, mask.float()) and y.grad is None
+    with torch.no_grad():
+        assert not select_rows(mask, x)[0].requires_grad

@@ -9,12 +9,13 @@ same quantities with F.grid_sample, elementwise torch ops and torch_scatter:
   DenseSdfGradient  lib/voxurf_fine.py:440-450 (neus_sdf_gradient, 'interpolate')
   NeusAlpha         lib/voxurf_fine.py:463-500 (neus_alpha_from_sdf_scatter)
   Alphas2Weights    lib/voxurf_fine.py:981-997
+  select_rows       the x[mask] compactions between the stages
   SegmentSum        torch_scatter.segment_coo(reduce='sum') at lib/voxurf_fine.py:753-777
 """
 import torch
 
 from . import render_utils_cuda as ru
-from ._lib import call, dtype_code, ptr, stream_of
+from ._lib import call, dtype_code, lib, ptr, stream_of
 from .total_variation_cuda import grid_geom
 
 
@@ -223,6 +224,64 @@ class SegmentSum(torch.autograd.Function):
         call("vx_segment_gather", dtype_code(gout), ptr(g2), ptr(index), ctx.shape[0], C,
              ctx.n_out, ptr(gsrc), stream_of(gout))
         return gsrc.reshape(ctx.shape), None, None
+
+
+def _row_words(t):
+    """32-bit words of a row of t (its first dimension's entries)."""
+    return t.element_size() * (t.numel() // max(t.shape[0], 1)) // 4
+
+
+def _copy_rows(mask, offsets, src, dst, transpose):
+    s, d = (torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64) for ts in (src, dst))
+    w = torch.tensor([_row_words(t) for t in (dst if transpose else src)], dtype=torch.int32)
+    call("vx_select_rows", ptr(mask), mask.shape[0], ptr(offsets), len(src), s.data_ptr(),
+         d.data_ptr(), w.data_ptr(), transpose, stream_of(mask))
+
+
+class _SelectRows(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, mask, *arrays):
+        n = mask.shape[0]
+        offsets = torch.empty(lib().vx_select_blocks(n), dtype=torch.int32, device=mask.device)
+        total = torch.empty(1, dtype=torch.int64, device=mask.device)
+        call("vx_select_count", ptr(mask), n, ptr(offsets), ptr(total), stream_of(mask))
+        src = [a.contiguous() for a in arrays]
+        m = int(total.item())
+        out = [torch.empty((m, *a.shape[1:]), dtype=a.dtype, device=a.device) for a in src]
+        if m:
+            _copy_rows(mask, offsets, src, out, 0)
+        ctx.mark_non_differentiable(*[o for o, g in zip(out, ctx.needs_input_grad[1:]) if not g])
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(mask, offsets)
+        return tuple(out)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, *gout):
+        mask, offsets = ctx.saved_tensors
+        res = [None] * len(gout)
+        src, dst = [], []
+        for k, g in enumerate(gout):
+            if g is None or not ctx.needs_input_grad[k + 1]:
+                continue
+            res[k] = torch.empty((mask.shape[0], *g.shape[1:]), dtype=g.dtype, device=g.device)
+            src.append(g.contiguous())
+            dst.append(res[k])
+        if src:
+            _copy_rows(mask, offsets, src, dst, 1)
+        return None, *res
+
+
+def select_rows(mask, *arrays):
+    """[a[mask] for a in arrays] (a boolean mask over the first dimension): the selected rows
+    are counted once and copied in one launch.  What the kernels do not take (an empty mask,
+    rows that are no 1 to 4096 whole words, more than eight arrays) is indexed."""
+    n = mask.shape[0]
+    if mask.dim() == 1 and mask.dtype == torch.bool and 0 < n < 1 << 31 and 0 < len(arrays) <= 8 and mask.is_cuda and all(
+            a.shape[0] == n and a.device == mask.device and a.numel() and
+            a.element_size() * (a.numel() // n) % 4 == 0 and _row_words(a) <= 4096 for a in arrays):
+        return _SelectRows.apply(mask.contiguous(), *arrays)
+    return tuple(a[mask] for a in arrays)
 
 
 def segment_coo(src, index, out=None, reduce="sum", dim_size=None):

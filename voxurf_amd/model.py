@@ -15,7 +15,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import render_utils_cuda as ru
-from .functional import (Alphas2Weights, NeusAlpha, SampleSdfs, SdfGradSample, segment_coo)
+from .functional import (Alphas2Weights, NeusAlpha, SampleSdfs, SdfGradSample, segment_coo,
+                         select_rows)
 from .grid import DenseGrid
 from .mlp import RgbNet
 from .scene import SceneConfig
@@ -50,11 +51,11 @@ class _VoxurfBase(nn.Module):
             rays_o.contiguous(), rays_d.contiguous(), self.xyz_min, self.xyz_max, 0.0, 1e9,
             stepdist)
         mask_inbbox = ~mask_outbbox
-        ray_pts, ray_id, step_id = ray_pts[mask_inbbox], ray_id[mask_inbbox], step_id[mask_inbbox]
+        ray_pts, ray_id, step_id = select_rows(mask_inbbox, ray_pts, ray_id, step_id)
         if getattr(self, "mask_cache", None) is not None:
             # known free space from the coarse geometry (lib/voxurf_fine.py:631-636)
             mask = self.mask_cache(ray_pts)
-            ray_pts, ray_id, step_id = ray_pts[mask], ray_id[mask], step_id[mask]
+            ray_pts, ray_id, step_id = select_rows(mask, ray_pts, ray_id, step_id)
             mask_outbbox[~mask_outbbox] |= ~mask
         return ray_pts, ray_id, step_id, mask_outbbox, N_steps
 
@@ -93,11 +94,12 @@ class VoxurfFine(_VoxurfBase):
         sdf, gradient = self.sdf_and_gradient(ray_pts)
         alpha = NeusAlpha.apply(viewdirs, ray_id, sdf, gradient, cfg.stepdist, self.inv_s)
         m = alpha > cfg.fast_color_thres
-        alpha, ray_id, ray_pts, gradient, step_id = alpha[m], ray_id[m], ray_pts[m], gradient[m], step_id[m]
+        alpha, ray_id, ray_pts, gradient, step_id = select_rows(m, alpha, ray_id, ray_pts, gradient,
+                                                                step_id)
         weights, alphainv_last = Alphas2Weights.apply(alpha, ray_id, N)
         m = weights > cfg.fast_color_thres
-        weights, ray_id, ray_pts, gradient, step_id = (weights[m], ray_id[m], ray_pts[m],
-                                                       gradient[m], step_id[m])
+        weights, ray_id, ray_pts, gradient, step_id = select_rows(m, weights, ray_id, ray_pts,
+                                                                  gradient, step_id)
         k0 = self.k0(ray_pts)
         normal = gradient / (gradient.norm(dim=-1, keepdim=True) + 1e-5)
         vemb = (viewdirs.unsqueeze(-1) * self.viewfreq).flatten(-2)
@@ -174,12 +176,12 @@ class Voxurf(_VoxurfBase):
         dist = cfg.stepdist
         alpha = NeusAlpha.apply(viewdirs, ray_id, sdf, gradient, dist, inv_s)
         m = alpha > cfg.fast_color_thres
-        alpha, ray_id, ray_pts, step_id = alpha[m], ray_id[m], ray_pts[m], step_id[m]
-        gradient, sdf = gradient[m], sdf[m]
+        alpha, ray_id, ray_pts, step_id, gradient, sdf = select_rows(m, alpha, ray_id, ray_pts,
+                                                                     step_id, gradient, sdf)
         weights, alphainv_last = Alphas2Weights.apply(alpha, ray_id, N)
         m = weights > cfg.fast_color_thres
-        weights, ray_id, ray_pts, step_id = weights[m], ray_id[m], ray_pts[m], step_id[m]
-        gradient, sdf = gradient[m], sdf[m]
+        weights, ray_id, ray_pts, step_id, gradient, sdf = select_rows(m, weights, ray_id, ray_pts,
+                                                                       step_id, gradient, sdf)
         k0 = self.k0(ray_pts)
         if k0.dim() == 1:
             k0 = k0[:, None]
@@ -268,7 +270,7 @@ class VoxurfCoarse(_VoxurfBase):
         alpha = NeusAlpha.apply(viewdirs, ray_id, sdf, gradient, cfg.stepdist, self.inv_s)
         weights, alphainv_last = Alphas2Weights.apply(alpha, ray_id, N)
         m = weights > cfg.fast_color_thres
-        ray_pts, ray_id, alpha = ray_pts[m], ray_id[m], alpha[m]
+        ray_pts, ray_id, alpha = select_rows(m, ray_pts, ray_id, alpha)
         weights, alphainv_last = Alphas2Weights.apply(alpha, ray_id, N)
         rgb = torch.sigmoid(self.k0(ray_pts))
         rgb_marched = segment_coo(weights.unsqueeze(-1) * rgb, ray_id,
