@@ -56,13 +56,12 @@ __device__ __forceinline__ void run_chunk(const FusedGeom& G, const float* start
   uint64_t mm = __ballot(cs.act);
   stop_lane = 64;
   cs.myT = 1.f;
+  const double through = 1.0 - (double)cs.alpha;
   while (mm) {
     const int k = __ffsll((unsigned long long)mm) - 1;
     mm &= mm - 1;
-    const float ak = __shfl(cs.alpha, k, 64);
     if (lane == k) cs.myT = T;
-    T = (float)((double)T * (1.0 - (double)ak));
-    if ((double)T < 1e-3) {
+    if (walk_step(T, through, k)) {
       stopped = true;
       stop_lane = k;
       break;

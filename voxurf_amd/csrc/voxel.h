@@ -70,6 +70,24 @@ __device__ __forceinline__ bool sample_point(const T* start, const T* dir, const
 }
 
 
+// Lane k's value (k the same in every lane).
+__device__ __forceinline__ double lane_value(double v, int k) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), k);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), k);
+  return __hiloint2double(hi, lo);
+}
+
+// One step of the transmittance recurrence T = (float)((double)T (1 - (double)alpha)), through
+// the sample of lane k (through: 1 - alpha, in double); true when the walk ends there,
+// (double)T < 1e-3 (1e-3f is the float next above 1e-3, so the same floats are below both).
+// Nothing but the multiplication and its roundings is in the chain from one step to the next,
+// and the branch is on a scalar: with a shuffle, the subtraction and a divergent branch in it a
+// step took 220 ns.
+__device__ __forceinline__ bool walk_step(float& T, double through, int k) {
+  T = (float)((double)T * lane_value(through, k));
+  return __ballot(T < 1e-3f) != 0;
+}
+
 // ---- trilinear lookups on dense grids -----------------------------------------------
 
 struct GridDesc {
