@@ -386,26 +386,6 @@ __global__ void __launch_bounds__(256) k_dense_grad_fwd(const T* __restrict__ s,
   out[2 * N + i] = (z > 0 && z < Z - 1) ? ((s[i + 1] - s[i - 1]) / (T)2) / vs : (T)0;
 }
 
-// Adjoint: gs[i] += sum_a (g_a[i - e_a] - g_a[i + e_a]) / 2 / vs over interior entries.
-template <typename T>
-__global__ void __launch_bounds__(256) k_dense_grad_bwd(const T* __restrict__ go, int X, int Y, int Z,
-                                                        T vs, T* __restrict__ gs) {
-#pragma clang fp contract(off)
-  const int z = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, x = blockIdx.z;
-  if (z >= Z) return;
-  const int64_t N = (int64_t)X * Y * Z;
-  const int64_t sx = (int64_t)Y * Z, sy = Z;
-  const int64_t i = x * sx + y * sy + z;
-  T acc = 0;
-  if (x - 1 > 0) acc += (go[i - sx] / (T)2) / vs;
-  if (x + 1 < X - 1) acc -= (go[i + sx] / (T)2) / vs;
-  if (y - 1 > 0) acc += (go[N + i - sy] / (T)2) / vs;
-  if (y + 1 < Y - 1) acc -= (go[N + i + sy] / (T)2) / vs;
-  if (z - 1 > 0) acc += (go[2 * N + i - 1] / (T)2) / vs;
-  if (z + 1 < Z - 1) acc -= (go[2 * N + i + 1] / (T)2) / vs;
-  gs[i] += acc;
-}
-
 // ---- total_variation_add_grad (lib/cuda/total_variation_kernel.cu:13-66) ----------
 // Weights arrive already divided by 6.  Axis weights follow the reference exactly: the
 // plain kernel uses wz on both the contiguous (k) and outermost (i) axes and wy on j;
@@ -586,6 +566,60 @@ static bool tv_rows(const GridDesc& g, const T* param, T* grad, const T* mask, f
     k_tv_rows<T, kMasked, 1><<<blocks, 256, 0, st>>>(param, grad, mask, g.X, g.Y, (int)row, (int)c_in,
                                                      (int)depth, wk, wj, wi, dense);
   return true;
+}
+
+// Adjoint of k_dense_grad_fwd: gs[i] += sum_a (g_a[i - e_a] - g_a[i + e_a]) / 2 / vs over
+// interior entries.  Bound by HBM: the three gradient grids read once and gs read and written
+// take 67 us at 256^3.  A thread per element, its block's neighbours in x and y on other XCDs,
+// read them again and took 143; vectors of a plane on 16 planes in turn, as k_tv_rows, 64.
+template <typename T, int V>
+__global__ void __launch_bounds__(256) k_dense_grad_bwd(const T* __restrict__ go, int X, int Y, int Z,
+                                                        int depth, T vs, T* __restrict__ gs) {
+#pragma clang fp contract(off)
+  const int64_t plane = (int64_t)Y * Z, N = X * plane;
+  const int64_t f = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+  if (f >= plane) return;
+  const int y = (int)(f / Z), z = (int)(f - (int64_t)y * Z);
+  const int x0 = blockIdx.y * depth, x1 = min(x0 + depth, X);
+  using Vec = TvVec<T, V>;
+  auto at = [&](const T* p) { return tv_load<T, V>(p, 0, V); };
+  Vec prev{}, cur{}, next{};
+  if (x0 > 0) prev = at(go + (x0 - 1) * plane + f);
+  cur = at(go + x0 * plane + f);
+  for (int x = x0; x < x1; ++x) {
+    const int64_t i = x * plane + f;
+    next = Vec{};
+    if (x + 1 < X) next = at(go + i + plane);
+    const Vec yl = y - 1 > 0 ? at(go + N + i - Z) : Vec{}, yh = y + 1 < Y - 1 ? at(go + N + i + Z) : Vec{};
+    const Vec zl = tv_load<T, V>(go + 2 * N + i - 1, 1 - z, V),
+              zh = tv_load<T, V>(go + 2 * N + i + 1, 0, Z - 1 - z);
+    Vec g = at(gs + i);
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      T acc = 0;
+      if (x - 1 > 0) acc += (prev.v[e] / (T)2) / vs;
+      if (x + 1 < X - 1) acc -= (next.v[e] / (T)2) / vs;
+      if (y - 1 > 0) acc += (yl.v[e] / (T)2) / vs;
+      if (y + 1 < Y - 1) acc -= (yh.v[e] / (T)2) / vs;
+      if (z + e - 1 > 0) acc += (zl.v[e] / (T)2) / vs;
+      if (z + e + 1 < Z - 1) acc -= (zh.v[e] / (T)2) / vs;
+      g.v[e] += acc;
+    }
+    __builtin_memcpy(gs + i, &g, sizeof(g));
+    prev = cur;
+    cur = next;
+  }
+}
+
+template <typename T>
+static void dense_grad_bwd(const T* go, int X, int Y, int Z, T vs, T* gs, hipStream_t st) {
+  const int v = Z % 4 == 0 ? 4 : 1;
+  const int64_t per_plane = cdiv((int64_t)Y * Z, 256 * v);
+  int64_t depth = per_plane * X / 2048;  // enough blocks for the chip first
+  depth = depth < 1 ? 1 : (depth > 16 ? 16 : depth);
+  const dim3 blocks((unsigned)per_plane, (unsigned)cdiv(X, depth));
+  if (v == 4) k_dense_grad_bwd<T, 4><<<blocks, 256, 0, st>>>(go, X, Y, Z, (int)depth, vs, gs);
+  else k_dense_grad_bwd<T, 1><<<blocks, 256, 0, st>>>(go, X, Y, Z, (int)depth, vs, gs);
 }
 
 // ---- SDF and unit normal on a lattice tile (lib/dvgo_ori.py:679-693 with the normal of
@@ -855,9 +889,8 @@ int vx_dense_sdf_gradient_bwd(int dtype, const void* gout, int X, int Y, int Z,
                               double voxel_size, void* gsdf, void* stream) {
   VX_CHECK_ARG(X >= 1 && Y >= 1 && Z >= 1, "dense gradient: bad shape");
   VX_CHECK_ARG(X <= 65535 && Y <= 65535, "dense gradient: X and Y must be <= 65535");
-  const dim3 grid((unsigned)cdiv(Z, 256), (unsigned)Y, (unsigned)X);
-  GRID_DISPATCH(dtype, k_dense_grad_bwd<scalar_t><<<grid, 256, 0, ST(stream)>>>(
-                           CP(gout), X, Y, Z, (scalar_t)voxel_size, MP(gsdf)));
+  GRID_DISPATCH(dtype, dense_grad_bwd<scalar_t>(CP(gout), X, Y, Z, (scalar_t)voxel_size, MP(gsdf),
+                                                ST(stream)));
   return launch_status("dense_sdf_gradient_bwd");
 }
 
