@@ -193,11 +193,81 @@ struct Taps {
   T w[kMaxTaps];
 };
 
-// Launched as a 3-D grid: (z chunks of 256 threads, y, x + X * channel).
-template <typename T>
+// V neighbouring elements of a plane on `depth` planes in turn, a load a tap: the taps along x
+// find their planes where this block has just read them.  Bound by HBM: 27 us an axis at 256^3
+// for one read and one write; a thread per element with the neighbours along x and y read by
+// blocks on other XCDs took 57, this 48.
+template <typename T, int V, int K>
 __global__ void __launch_bounds__(256) k_smooth_axis(const T* __restrict__ in, T* __restrict__ out,
-                                                     int C, int X, int Y, int Z, int axis,
-                                                     Taps<T> taps, int k, int transpose) {
+                                                     int X, int Y, int Z, int depth, int axis,
+                                                     Taps<T> taps) {
+  const int64_t plane = (int64_t)Y * Z, f = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+  if (f >= plane) return;
+  const int y = (int)(f / Z), z = (int)(f - (int64_t)y * Z);
+  const int x0 = blockIdx.y * depth, x1 = min(x0 + depth, X);
+  constexpr int r = K / 2;
+  struct Vec {
+    T v[V];
+  };
+  in += (int64_t)blockIdx.z * X * plane;
+  out += (int64_t)blockIdx.z * X * plane;
+  for (int x = x0; x < x1; ++x) {
+    Vec a[K];
+#pragma unroll
+    for (int t = 0; t < K; ++t) {
+      if (axis == 2) {
+        const T* line = in + x * plane + (f - z);
+        if (z + t - r >= 0 && z + t - r + V <= Z) {
+          __builtin_memcpy(&a[t], line + (z + t - r), sizeof(Vec));
+        } else {
+#pragma unroll
+          for (int e = 0; e < V; ++e) a[t].v[e] = line[clampi(z + e + t - r, 0, Z - 1)];
+        }
+      } else {
+        const int64_t at = axis == 1 ? x * plane + (int64_t)clampi(y + t - r, 0, Y - 1) * Z + z
+                                     : clampi(x + t - r, 0, X - 1) * plane + f;
+        __builtin_memcpy(&a[t], in + at, sizeof(Vec));
+      }
+    }
+    Vec o;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      T acc = 0;
+#pragma unroll
+      for (int t = 0; t < K; ++t) acc += taps.w[t] * a[t].v[e];
+      o.v[e] = acc;
+    }
+    __builtin_memcpy(out + x * plane + f, &o, sizeof(Vec));
+  }
+}
+
+template <typename T, int K>
+static void smooth_axis(const T* in, T* out, int C, int X, int Y, int Z, int axis,
+                        const Taps<T>& taps, hipStream_t st) {
+  const int v = Z % 4 == 0 ? 4 : 1;
+  const int64_t per_plane = cdiv((int64_t)Y * Z, 256 * v);
+  int64_t depth = per_plane * X * C / 2048;  // enough blocks for the chip first
+  depth = depth < 1 ? 1 : (depth > 16 ? 16 : depth);
+  const dim3 grid((unsigned)per_plane, (unsigned)cdiv(X, depth), (unsigned)C);
+  if (v == 4) k_smooth_axis<T, 4, K><<<grid, 256, 0, st>>>(in, out, X, Y, Z, (int)depth, axis, taps);
+  else k_smooth_axis<T, 1, K><<<grid, 256, 0, st>>>(in, out, X, Y, Z, (int)depth, axis, taps);
+}
+
+template <typename T>
+static void smooth_axis(const T* in, T* out, int C, int X, int Y, int Z, int axis,
+                        const Taps<T>& taps, int k, hipStream_t st) {
+  if (k == 1) smooth_axis<T, 1>(in, out, C, X, Y, Z, axis, taps, st);
+  else if (k == 3) smooth_axis<T, 3>(in, out, C, X, Y, Z, axis, taps, st);
+  else if (k == 5) smooth_axis<T, 5>(in, out, C, X, Y, Z, axis, taps, st);
+  else if (k == 7) smooth_axis<T, 7>(in, out, C, X, Y, Z, axis, taps, st);
+  else smooth_axis<T, 9>(in, out, C, X, Y, Z, axis, taps, st);
+}
+
+// The adjoint.  Launched as a 3-D grid: (z chunks of 256 threads, y, x + X * channel).
+template <typename T>
+__global__ void __launch_bounds__(256) k_smooth_axis_bwd(const T* __restrict__ in, T* __restrict__ out,
+                                                         int C, int X, int Y, int Z, int axis,
+                                                         Taps<T> taps, int k) {
   const int z = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
   const int x = blockIdx.z % X, c = blockIdx.z / X;
   if (z >= Z) return;
@@ -208,29 +278,25 @@ __global__ void __launch_bounds__(256) k_smooth_axis(const T* __restrict__ in, T
   const int r = k / 2;
   const T* line = in + (i - (int64_t)u * stride);
   T acc = 0;
-  if (!transpose) {
-    for (int t = 0; t < k; ++t) acc += taps.w[t] * line[(int64_t)clampi(u + t - r, 0, n - 1) * stride];
-  } else {
-    for (int t = 0; t < k; ++t) {
-      // the v whose tap t lands on u
-      int lo, hi;
-      if (u == 0 && u == n - 1) {
-        lo = 0;
-        hi = 0;
-      } else if (u == 0) {
-        lo = 0;
-        hi = min(n - 1, r - t);
-      } else if (u == n - 1) {
-        lo = max(0, n - 1 - t + r);
-        hi = n - 1;
-      } else {
-        lo = hi = u - t + r;
-        if (lo < 0 || lo > n - 1) continue;
-      }
-      T s = 0;
-      for (int v = lo; v <= hi; ++v) s += line[(int64_t)v * stride];
-      acc += taps.w[t] * s;
+  for (int t = 0; t < k; ++t) {
+    // the v whose tap t lands on u
+    int lo, hi;
+    if (u == 0 && u == n - 1) {
+      lo = 0;
+      hi = 0;
+    } else if (u == 0) {
+      lo = 0;
+      hi = min(n - 1, r - t);
+    } else if (u == n - 1) {
+      lo = max(0, n - 1 - t + r);
+      hi = n - 1;
+    } else {
+      lo = hi = u - t + r;
+      if (lo < 0 || lo > n - 1) continue;
     }
+    T s = 0;
+    for (int v = lo; v <= hi; ++v) s += line[(int64_t)v * stride];
+    acc += taps.w[t] * s;
   }
   out[i] = acc;
 }
@@ -348,12 +414,16 @@ int vx_smooth3d(int dtype, const void* in, void* out, void* tmp, int C, int X, i
     const scalar_t* src = (const scalar_t*)in;
     const dim3 grid((unsigned)cdiv(Z, 256), (unsigned)Y, (unsigned)((int64_t)X * C));
     // z into out, y into tmp, x into out
-    k_smooth_axis<scalar_t><<<grid, 256, 0, st>>>(src, (scalar_t*)out, C, X, Y, Z, 2, w, k,
-                                                  transpose);
-    k_smooth_axis<scalar_t><<<grid, 256, 0, st>>>((const scalar_t*)out, (scalar_t*)tmp, C, X, Y, Z,
-                                                  1, w, k, transpose);
-    k_smooth_axis<scalar_t><<<grid, 256, 0, st>>>((const scalar_t*)tmp, (scalar_t*)out, C, X, Y, Z,
-                                                  0, w, k, transpose);
+    scalar_t *o = (scalar_t*)out, *t = (scalar_t*)tmp;
+    if (transpose) {
+      k_smooth_axis_bwd<scalar_t><<<grid, 256, 0, st>>>(src, o, C, X, Y, Z, 2, w, k);
+      k_smooth_axis_bwd<scalar_t><<<grid, 256, 0, st>>>((const scalar_t*)o, t, C, X, Y, Z, 1, w, k);
+      k_smooth_axis_bwd<scalar_t><<<grid, 256, 0, st>>>((const scalar_t*)t, o, C, X, Y, Z, 0, w, k);
+    } else {
+      smooth_axis<scalar_t>(src, o, C, X, Y, Z, 2, w, k, st);
+      smooth_axis<scalar_t>((const scalar_t*)o, t, C, X, Y, Z, 1, w, k, st);
+      smooth_axis<scalar_t>((const scalar_t*)t, o, C, X, Y, Z, 0, w, k, st);
+    }
   });
   return launch_status("smooth3d");
 }
