@@ -117,33 +117,62 @@ def test_sdf_gradient_without_neighbour_values(dev):
 def test_total_variation_rows(dev, C, inner, shape, masked, dense):
     g = torch.Generator().manual_seed(C + sum(shape))
     X, Y, Z = shape
-    # the strided kernel gets the same values in rows one element longer
     full = (X, Y, Z, C) if inner else (C, X, Y, Z)
     val = [torch.randn(full, generator=g) for _ in range(3)]
     val[1][torch.rand(full, generator=g) < 0.5] = 0
     val[2] = (val[2] > 0).float()
+    res = [_tv(dev, val, inner, masked, dense, (0.3, 0.5, 0.7), long) for long in (False, True)]
+    assert torch.equal(*res)
 
-    def view(t, long):
+
+def _tv(dev, val, inner, masked, dense, w, long):
+    """The gradient val[1] (parameters val[0], mask val[2]) with the total variation's added;
+    long: in rows one element longer, which only the strided kernel takes."""
+    full = val[0].shape
+
+    def view(t):
         if long:
-            w = torch.zeros((*full[:-1], full[-1] + 1))
+            w = torch.zeros((*full[:-1], full[-1] + 1), dtype=t.dtype)
             w[..., :full[-1]] = t
             t = w.to(dev)[..., :full[-1]]
         else:
             t = t.to(dev)
         return (t.permute(3, 0, 1, 2) if inner else t)[None]
 
-    res = []
-    for long in (False, True):
-        p, gr, m = (view(v, long) for v in val)
-        geom = grid_geom(p)
-        if masked:
-            call("vx_total_variation_add_grad_new", 0, ptr(p), ptr(gr), ptr(m), geom.data_ptr(), 0.3,
-                 0.5, 0.7, dense, stream_of(p))
-        else:
-            call("vx_total_variation_add_grad", 0, ptr(p), ptr(gr), geom.data_ptr(), 0.3, 0.5, 0.7,
-                 dense, stream_of(p))
-        res.append(gr.contiguous())
-    assert torch.equal(*res)
+    p, gr, m = (view(v) for v in val)
+    geom = grid_geom(p)
+    args = (dtype_code(p), ptr(p), ptr(gr), *([ptr(m)] if masked else []), geom.data_ptr(), *w, dense,
+            stream_of(p))
+    call("vx_total_variation_add_grad_new" if masked else "vx_total_variation_add_grad", *args)
+    return gr.contiguous()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("C,inner", [(1, False), (3, False), (3, True), (4, True)])
+@pytest.mark.parametrize("shape", [(6, 5, 8), (5, 4, 7)])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("dense", [0, 1])
+def test_total_variation_that_cancels(dev, dtype, C, inner, shape, masked, dense):
+    """Whole numbers (differences clamped to -1, 0 or 1, weights of 6 / 6), the gradient of every
+    other element minus its term: the sums are exact, and an element that had a gradient holds
+    exactly zero afterwards; one without stays as it is where only those are taken."""
+    g = torch.Generator().manual_seed(C + sum(shape))
+    X, Y, Z = shape
+    full = (X, Y, Z, C) if inner else (C, X, Y, Z)
+    p = torch.randint(-3, 4, full, generator=g).to(dtype)
+    mask = (torch.rand(full, generator=g) < 0.7).to(dtype)
+    zero = torch.zeros(full, dtype=dtype)
+    w = (6.0, 6.0, 6.0)
+    term = _tv(dev, [p, zero, mask], inner, masked, 1, w, True).cpu()
+    term = (term[0].permute(1, 2, 3, 0) if inner else term[0]).contiguous()
+    own = torch.rand(full, generator=g) < 0.5
+    assert int((own & (term != 0)).sum()) > 10
+    val = [p, torch.where(own, -term, zero), mask]
+    res = [_tv(dev, val, inner, masked, dense, w, long) for long in (False, True)]
+    want = torch.where(own, zero, term if dense else zero)
+    want = (want.permute(3, 0, 1, 2) if inner else want)[None].to(dev)
+    for r in res:
+        assert torch.equal(r, want)
 
 
 @pytest.mark.parametrize("tile,origin,res", [(1, (0, 0, 0), 8), (5, (3, 0, 2), 40), (63, (1, 4, 0), 70),

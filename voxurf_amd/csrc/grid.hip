@@ -485,10 +485,12 @@ __global__ void __launch_bounds__(256) k_tv_rows(const T* __restrict__ param, T*
       if (kMasked) mnext = at(mm, x + 1);
     }
     Vec g = tv_load<T, V>(gm + x * plane, 0, V);
-    bool any = dense;
+    // the elements that take the term, told from the gradient before it is added: a sum that
+    // cancels to zero is stored like any other
+    unsigned take = 0u;
 #pragma unroll
-    for (int e = 0; e < V; ++e) any = any || g.v[e] != (T)0;
-    if (any) {
+    for (int e = 0; e < V; ++e) take |= (dense || g.v[e] != (T)0 ? 1u : 0u) << e;
+    if (take) {
       const T* p = pm + x * plane;
       const T* m = kMasked ? mm + x * plane : nullptr;
       const Vec zl = tv_load<T, V>(p - C_in, below, V), zh = tv_load<T, V>(p + C_in, 0, above);
@@ -503,7 +505,7 @@ __global__ void __launch_bounds__(256) k_tv_rows(const T* __restrict__ param, T*
       }
 #pragma unroll
       for (int e = 0; e < V; ++e) {
-        if (!dense && g.v[e] == (T)0) continue;
+        if (!(take >> e & 1u)) continue;
         const T c = cur.v[e];
         float add = 0;
         auto term = [&](bool has, T nb, T mnb, float w) {
@@ -529,7 +531,7 @@ __global__ void __launch_bounds__(256) k_tv_rows(const T* __restrict__ param, T*
       } else {
 #pragma unroll
         for (int e = 0; e < V; ++e)
-          if (g.v[e] != (T)0) o[e] = g.v[e];
+          if (take >> e & 1u) o[e] = g.v[e];
       }
     }
     prev = cur;
