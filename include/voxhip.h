@@ -556,15 +556,11 @@ int vx_mlp_layer_fwd(int prec, int kt, int k_in, int last, const void* in, int i
                      int64_t M, const void* wpk, const float* bias, void* out, int out_stride,
                      const float* w3, const float* b3, float* logits, const int64_t* M_dev,
                      uint32_t* mask_bits, void* stream);
-/* The whole network in one launch, FP32 accuracy from two-way FP16 splits of scaled rows and
- * weights (three MFMA products per FP32 product).  vx_mlp_pack_half packs the hidden layers'
- * weights (w_ptrs: host array of n_hidden device addresses, 1..4 layers, width 192, input
- * width k_in0 <= 96) into vx_mlp_pack_half_bytes bytes (16-byte aligned; -1: bad sizes). */
-int64_t vx_mlp_pack_half_bytes(int n_hidden, int k_in0);
-int vx_mlp_pack_half(int n_hidden, const int64_t* w_ptrs, int k_in0, void* out, void* stream);
-/* logits [M, 3] of X [M, xs] (float32 rows padded to 64 columns for k_in0 <= 64, else 96;
- * finite past k_in0) without keeping activations; biases: host array of n_hidden device
- * addresses. */
+/* The whole network in one launch without keeping activations: the logits [M, 3] that
+ * vx_mlp_layer_fwd and vx_mlp_logits give with prec 2, bit for bit, for X [M, xs] (float32 rows
+ * padded to 64 columns for k_in0 <= 64, else 96; finite past k_in0), 1..4 hidden layers of
+ * width 192 and input width k_in0 <= 96; packed: vx_mlp_pack_net's output for prec 2; biases:
+ * host array of n_hidden device addresses. */
 int vx_mlp_net_fwd(int n_hidden, int k_in0, const float* X, int xs, int64_t M, const void* packed,
                    const int64_t* biases, const float* w3, const float* b3, float* logits,
                    const int64_t* M_dev, void* stream);

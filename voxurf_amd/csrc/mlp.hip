@@ -673,155 +673,91 @@ __global__ void __launch_bounds__(kLayerThreads) k_mlp_layer_split(
   }
 }
 
-// ---- the whole network in one pass, FP32 through two-way FP16 splits --------------------
-// Two things bound the layer-at-a-time passes above: every activation row goes to HBM and
-// back between the layers (at 1.4 M rows a 131,072-ray render spent 2.3 ms on 4.3 GB of
-// them), and six BF16 products per FP32 product.  For a forward whose activations
-// nobody reads afterwards (no backward to come) both go:
+// ---- the whole network in one pass, FP32 through BF16 splits ------------------------------
+// A layer at a time, every activation row goes to HBM and back between the layers: at 1.4 M
+// rows a 131,072-ray render spent 2.3 ms on 4.3 GB of them.  For a forward whose activations
+// nobody reads afterwards (no backward to come) a wave keeps a tile of 32 rows in registers
+// through all the layers: a layer's accumulators (row = feature, column = sample) hold, after
+// bias and ReLU, exactly the next layer's B operands.  What moves is the weights: a layer's
+// 32-feature slab (all 192 outputs, three parts, 36.9 KB) is staged in one of three LDS
+// buffers, loaded from L2 two slabs ahead, and the eight waves of a workgroup (two per SIMD,
+// 256 registers each) multiply it together, one barrier a slab.  Every output element's MFMAs,
+// bias, ReLU and logit sums are those of k_mlp_layer_split and k_mlp_logits in the same order,
+// so the logits are theirs bit for bit, with a gradient to follow or without.
 //
-// A wave keeps a tile of 32 rows in registers through all the layers: a layer's accumulators
-// (row = feature, column = sample) hold, after bias and ReLU or mask, exactly the next
-// layer's B operands.  What moves is the weights: a layer's 32-feature slab (all 192
-// outputs, 24.6 KB) is staged in one of three LDS buffers, loaded from L2 two slabs ahead, and
-// the waves of a workgroup multiply it together, one barrier a slab.
-//
-// With whole rows in registers a row can be scaled: by the power of two that brings its
-// largest entry into [2^14, 2^15), and each output feature's weights likewise.  A scaled x is
-// then x0 + x1 with x0 = fp16(x) and x1 = fp16(x - x0) to within 2^-23 |x| (and 2^-39 of the
-// row's largest entry: fp16 keeps 2^-24 as its smallest step), a product x w is
-// x0 w0 + x0 w1 + x1 w0 to within 2^-22, and a 16-deep step takes three MFMAs instead of six
-// (this way to a single-precision product from half-precision ones is Ootomo and Yokota's,
-// "Recovering single precision accuracy from Tensor Cores while surpassing the FP32
-// theoretical peak performance", 2022).  The sum's rounding dominates either way, and with
-// half the MFMAs there is less of it: errors against float64 are no larger than the six
-// products' (measured in the tests over the widths and row counts in use).
-//
-// Matrix products reach 1,212 TFLOP/s in bf16 on this card; the six-product form of this
-// kernel ran 1.4 M rows in 1,450 us (961), this one in 803 us.
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
+// Bound by the matrix cores: 1.4 M rows of 42 columns in 1,186 us, 1,175 TFLOP/s of BF16
+// products where a large product reaches 1,212 (the layers' passes: 2,300 us).  Up to 256 rows
+// a CU (65,536) it is one round of 14 slabs, 45 us from one row on.  Three products of two
+// FP16 parts with a scale a row took 803 us, but kept 22 bits of an operand instead of 24, and
+// fewer of entries far below their row's largest (beside one of 1e8 with zero weights: 6e-6
+// off float64 where this is 4e-7), so the parts are the layers' three.
 constexpr int kNetMaxHidden = 4;
 constexpr int kNetWaves = 8;                // two per SIMD
-constexpr int kNetRuns = 24;                // 1 KB runs of a slab: [tile][step][part]
-constexpr int kNetStage = kNetRuns / kNetWaves;
-
-// Exponent-only scale that brings m into [2^14, 2^15), and its inverse.  (m = 0 and numbers
-// below 2^-112 take the largest scale.)
-__device__ __forceinline__ void half_scale(float m, float& s, float& inv) {
-  int e = (int)(__float_as_uint(m) >> 23 & 255u) - 127;
-  e = e < -112 ? -112 : e;
-  s = __uint_as_float((uint32_t)(127 + 14 - e) << 23);
-  inv = __uint_as_float((uint32_t)(127 - 14 + e) << 23);
-}
-
-__device__ __forceinline__ void split2(float x, _Float16& p0, _Float16& p1) {
-  p0 = (_Float16)x;
-  p1 = (_Float16)(x - (float)p0);
-}
-
-// Packed forward operands: layer li at half offset w[li], f16x8 vector
-// ((to * S + s) * 2 + part) * 64 + lane holding the eight k of step s (as pack_bf16_value),
-// then the inverse scales, 192 floats a layer.
-struct HalfNet {
-  PackSeg seg[kNetMaxHidden];
-  int64_t scales;  // offset of the inverse scales, in halves
-};
-
-// One wave per (layer, output feature i of the operand).
-__global__ void __launch_bounds__(256) k_pack_half(HalfNet net, _Float16* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), li = blockIdx.y;
-  const PackSeg sg = net.seg[li];
-  float v[3];
-  float m = 0.f;
-#pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    const int k = lane + 64 * j;
-    v[j] = 0.f;
-    if (k < sg.k_in) v[j] = sg.W[i * sg.k_in + k];
-    m = fmaxf(m, fabsf(v[j]));
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  float s, inv;
-  half_scale(m, s, inv);
-  if (lane == 0) reinterpret_cast<float*>(out + net.scales)[li * kWidth + i] = inv;
-  const int S = 2 * sg.kt;
-#pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    const int k = lane + 64 * j;
-    if (k >= 32 * sg.kt) continue;
-    const int r = k & 31, h = r >> 2 & 1, a = 4 * (r >> 3) + (r & 3);  // dfeat(k / 32, a, h) = k
-    const int st = 2 * (k >> 5) + (a >> 3);
-    _Float16 p0, p1;
-    split2(v[j] * s, p0, p1);
-    _Float16* o = out + sg.offset + ((((int64_t)(i >> 5) * S + st) * 2) * 64 + (i & 31) + 32 * h) * 8 + (a & 7);
-    o[0] = p0;
-    o[64 * 8] = p1;
-  }
-}
+constexpr int kNetRuns = 36;                // 1 KB runs of a slab: [tile][step][part]
+constexpr int kNetStage = (kNetRuns + kNetWaves - 1) / kNetWaves;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct NetArgs {
   const float* in;
-  int in_stride, n_hidden, k_in;
+  int in_stride, n_hidden;
   int64_t M;
   const int64_t* Md;
-  const f16x8* w[kNetMaxHidden];
-  const float* ws;  // inverse scales [n_hidden][192]
+  const bf16x8* w[kNetMaxHidden];
   const float* b[kNetMaxHidden];
   const float* w3;
   const float* b3;
   float* logits;
 };
 
-// Slab (step pair t) of a layer with `steps` 16-deep steps: runs of 64 vectors, four an
-// output tile, run wave + kNetWaves k in each wave's k-th register.
-__device__ __forceinline__ void net_load(u32x4 (&v)[kNetStage], const f16x8* __restrict__ w,
+// Slab (step pair t) of a layer with `steps` 16-deep steps: runs of 64 vectors, six an output
+// tile, run wave + kNetWaves k in each wave's k-th register (a run past the slab reads its
+// last one and is not stored).
+__device__ __forceinline__ void net_load(u32x4 (&v)[kNetStage], const bf16x8* __restrict__ w,
                                          int steps, int t, int wave, int lane) {
 #pragma unroll
   for (int k = 0; k < kNetStage; ++k) {
-    const int run = wave + kNetWaves * k;
-    v[k] = reinterpret_cast<const u32x4*>(w)[((run >> 2) * steps + 2 * t) * 128 + (run & 3) * 64 + lane];
+    const int run = min(wave + kNetWaves * k, kNetRuns - 1), to = run / 6;
+    v[k] = reinterpret_cast<const u32x4*>(w)[(to * steps + 2 * t) * 192 + (run - 6 * to) * 64 + lane];
   }
 }
 
-__device__ __forceinline__ void net_store(const u32x4 (&v)[kNetStage], f16x8* lw, int wave, int lane) {
+__device__ __forceinline__ void net_store(const u32x4 (&v)[kNetStage], bf16x8* lw, int wave, int lane) {
 #pragma unroll
-  for (int k = 0; k < kNetStage; ++k)
-    reinterpret_cast<u32x4*>(lw)[(wave + kNetWaves * k) * 64 + lane] = v[k];
+  for (int k = 0; k < kNetStage; ++k) {
+    const int run = wave + kNetWaves * k;
+    if (run < kNetRuns) reinterpret_cast<u32x4*>(lw)[run * 64 + lane] = v[k];
+  }
 }
 
-// One slab into the accumulators: acc[to] += W slab x (s x) (x: the 16 features of the slab a
-// lane holds of its row, s the row's scale).  QN as in split_slab.  Two output tiles at a
-// time: their independent MFMAs alternate.
+// One slab into the accumulators: acc[to] += W slab x x (the 16 features of the slab a lane
+// holds of its row).  QN as in split_slab.  Two output tiles at a time: their independent
+// MFMAs alternate.
 template <int QN>
-__device__ __forceinline__ void net_slab(f32x16 (&acc)[6], const f32x16& x, float s,
-                                         const f16x8* lw, int lane) {
+__device__ __forceinline__ void net_slab(f32x16 (&acc)[6], const f32x16& x, const bf16x8* lw,
+                                         int lane) {
 #pragma unroll
   for (int q = 0; q < QN; ++q) {
-    f16x8 b0, b1;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      _Float16 q0, q1;
-      split2(x[8 * q + e] * s, q0, q1);
-      b0[e] = q0;
-      b1[e] = q1;
-    }
+    bf16x8 b0, b1, b2;
+    split8(make_float4(x[8 * q], x[8 * q + 1], x[8 * q + 2], x[8 * q + 3]),
+           make_float4(x[8 * q + 4], x[8 * q + 5], x[8 * q + 6], x[8 * q + 7]), b0, b1, b2);
     constexpr int P = 2;
 #pragma unroll
     for (int to = 0; to < 6; to += P) {
-      f16x8 a0[P], a1[P];
+      bf16x8 a0[P], a1[P], a2[P];
 #pragma unroll
       for (int i = 0; i < P; ++i) {
-        const f16x8* a = lw + (((to + i) * 2 + q) * 2) * 64 + lane;
+        const bf16x8* a = lw + (((to + i) * 2 + q) * 3) * 64 + lane;
         a0[i] = a[0];
         a1[i] = a[64];
+        a2[i] = a[128];
       }
-      // smallest terms first
+      // smallest terms first, as split_slab
 #define NET_MFMA(A, B)                                                                    \
   _Pragma("unroll") for (int i = 0; i < P; ++i)                                           \
-    acc[to + i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[i], B, acc[to + i], 0, 0, 0);
+    acc[to + i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[i], B, acc[to + i], 0, 0, 0);
+      NET_MFMA(a2, b0)
+      NET_MFMA(a1, b1)
+      NET_MFMA(a0, b2)
       NET_MFMA(a1, b0)
       NET_MFMA(a0, b1)
       NET_MFMA(a0, b0)
@@ -837,24 +773,12 @@ __device__ __forceinline__ void net_zero(f32x16 (&acc)[6]) {
     for (int v = 0; v < 16; ++v) acc[to][v] = 0.f;
 }
 
-// Largest |entry| of the lane's row over the first NT slabs (both lane halves).
-template <int NT>
-__device__ __forceinline__ float row_max(const f32x16 (&x)[6]) {
-  float m[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) m[v & 3] = fmaxf(m[v & 3], fabsf(x[t][v]));
-  const float r = fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3]));
-  return fmaxf(r, __shfl_xor(r, 32, 64));
-}
-
 // The slab after next on its way while this one is multiplied, then into the buffer that the
 // slab before this one has left.
 #define NET_STEP(T, QN)                                                                  \
   {                                                                                       \
     load();                                                                               \
-    net_slab<QN>(acc, x[T], sc, lw[cur], lane);                                           \
+    net_slab<QN>(acc, x[T], lw[cur], lane);                                               \
     net_store(stage, lw[cur == 0 ? 2 : cur - 1], wave, lane);                             \
     cur = cur == 2 ? 0 : cur + 1;                                                         \
     __syncthreads();                                                                      \
@@ -864,8 +788,8 @@ __device__ __forceinline__ float row_max(const f32x16 (&x)[6]) {
 // packed width), KQ0: its 16-deep steps with weights that are not all zero.
 template <int KT0, int KQ0>
 __global__ void __launch_bounds__(64 * kNetWaves) k_mlp_net_fwd(NetArgs a) {
-  __shared__ f16x8 lw[3][kNetRuns * 64];
-  __shared__ float lb[kNetMaxHidden][2][kWidth];  // bias, inverse weight scale
+  __shared__ bf16x8 lw[3][kNetRuns * 64];
+  __shared__ float lb[kNetMaxHidden][kWidth];
   __shared__ float l3[3 * kWidth + 4];
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, rl = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -874,10 +798,7 @@ __global__ void __launch_bounds__(64 * kNetWaves) k_mlp_net_fwd(NetArgs a) {
   const int64_t rounds = (M + kRows - 1) / kRows;
   if ((int64_t)blockIdx.x >= rounds) return;
   for (int li = 0; li < a.n_hidden; ++li)
-    if (tid < kWidth) {
-      lb[li][0][tid] = a.b[li][tid];
-      lb[li][1][tid] = a.ws[li * kWidth + tid];
-    }
+    if (tid < kWidth) lb[li][tid] = a.b[li][tid];
   for (int i = tid; i < 3 * kWidth + 3; i += 64 * kNetWaves)
     l3[i] = i < 3 * kWidth ? a.w3[i] : a.b3[i - 3 * kWidth];
   // the slab to load next: its layer and step pair
@@ -898,7 +819,6 @@ __global__ void __launch_bounds__(64 * kNetWaves) k_mlp_net_fwd(NetArgs a) {
   int cur = 0;
   f32x16 x[6];    // the layer's input, slab by slab
   f32x16 acc[6];
-  float sc, inv;
   __syncthreads();
   for (int64_t round = blockIdx.x; round < rounds; round += gridDim.x) {
     const int64_t r = round * kRows + wave * 32 + rl;
@@ -914,32 +834,23 @@ __global__ void __launch_bounds__(64 * kNetWaves) k_mlp_net_fwd(NetArgs a) {
           x[t][4 * u + 2] = v.z;
           x[t][4 * u + 3] = v.w;
         }
-      // columns past the weights' (any finite values) must not set the row's scale
-#pragma unroll
-      for (int t = 0; t < KT0; ++t)
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          if (dfeat(t, v, h) >= a.k_in) x[t][v] = 0.f;
-      half_scale(row_max<KT0>(x), sc, inv);
     }
-    // scales, bias and ReLU: the next layer's input (and the logits' at the end)
+    // bias and ReLU: the next layer's input (and the logits' at the end)
     auto finish = [&](int li) __attribute__((always_inline)) {
 #pragma unroll
       for (int to = 0; to < 6; ++to) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const float4 b4 = *reinterpret_cast<const float4*>(&lb[li][0][32 * to + 8 * u + 4 * h]);
-          const float4 s4 = *reinterpret_cast<const float4*>(&lb[li][1][32 * to + 8 * u + 4 * h]);
-          const float bv[4] = {b4.x, b4.y, b4.z, b4.w}, sv[4] = {s4.x, s4.y, s4.z, s4.w};
+          const float4 b4 = *reinterpret_cast<const float4*>(&lb[li][32 * to + 8 * u + 4 * h]);
+          const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float v = fmaf(acc[to][4 * u + e] * inv, sv[e], bv[e]);
+            const float v = acc[to][4 * u + e] + bv[e];
             x[to][4 * u + e] = v > 0.f ? v : 0.f;
           }
         }
         __builtin_amdgcn_sched_barrier(0);  // (or the reads of all tiles come first, and spill)
       }
-      half_scale(row_max<6>(x), sc, inv);
     };
     net_zero(acc);
 #pragma unroll
@@ -1710,59 +1621,31 @@ int vx_mlp_layer_fwd(int prec, int kt, int k_in, int last, const void* in, int i
   return launch_status("mlp_layer_fwd");
 }
 
-static int half_net(HalfNet& net, int n_hidden, int k_in0, const int64_t* w_ptrs) {
-  VX_CHECK_ARG(n_hidden >= 1 && n_hidden <= kNetMaxHidden, "mlp_net: 1..%d hidden layers",
-               kNetMaxHidden);
-  VX_CHECK_ARG(k_in0 >= 1 && k_in0 <= 96, "mlp_net: input width must be 1..96");
-  PackNet all;
-  int64_t total = 0, off = 0;
-  pack_net_segments(n_hidden, k_in0, w_ptrs, &all, &total);
-  for (int li = 0; li < n_hidden; ++li) {
-    net.seg[li] = all.seg[2 * li];
-    net.seg[li].offset = off;
-    off += 2 * vx_mlp_pack_elems(net.seg[li].kt, net.seg[li].nto);
-  }
-  net.scales = off;
-  return VX_OK;
-}
-
-int64_t vx_mlp_pack_half_bytes(int n_hidden, int k_in0) {
-  HalfNet net;
-  if (half_net(net, n_hidden, k_in0, nullptr)) return -1;
-  return 2 * net.scales + 4 * (int64_t)n_hidden * kWidth;
-}
-
-int vx_mlp_pack_half(int n_hidden, const int64_t* w_ptrs, int k_in0, void* out, void* stream) {
-  VX_CHECK_ARG(w_ptrs && out, "mlp_pack_half: missing argument");
-  HalfNet net;
-  if (int e = half_net(net, n_hidden, k_in0, w_ptrs)) return e;
-  k_pack_half<<<dim3(kWidth / 4, (unsigned)n_hidden), 256, 0, (hipStream_t)stream>>>(net, (_Float16*)out);
-  return launch_status("mlp_pack_half");
-}
-
 int vx_mlp_net_fwd(int n_hidden, int k_in0, const float* X, int xs, int64_t M, const void* packed,
                    const int64_t* biases, const float* w3, const float* b3, float* logits,
                    const int64_t* M_dev, void* stream) {
+  VX_CHECK_ARG(n_hidden >= 1 && n_hidden <= kNetMaxHidden, "mlp_net_fwd: 1..%d hidden layers",
+               kNetMaxHidden);
+  VX_CHECK_ARG(k_in0 >= 1 && k_in0 <= 96, "mlp_net_fwd: input width must be 1..96");
   const int kt0 = k_in0 <= 64 ? 2 : 3;
-  HalfNet net;
-  if (int e = half_net(net, n_hidden, k_in0, nullptr)) return e;
   VX_CHECK_ARG(M >= 0, "mlp_net_fwd: M < 0");
   VX_CHECK_ARG(xs >= 32 * kt0 && xs % 4 == 0, "mlp_net_fwd: rows must be padded to 64 or 96");
   if (M == 0) return VX_OK;
   VX_CHECK_ARG(X && packed && biases && w3 && b3 && logits, "mlp_net_fwd: null pointer");
+  PackNet net;
+  int64_t total = 0;
+  pack_net_segments(n_hidden, k_in0, nullptr, &net, &total);
   NetArgs a{};
   a.in = X;
   a.in_stride = xs;
   a.n_hidden = n_hidden;
-  a.k_in = k_in0;
   a.M = M;
   a.Md = M_dev;
-  a.ws = (const float*)((const _Float16*)packed + net.scales);
   a.w3 = w3;
   a.b3 = b3;
   a.logits = logits;
   for (int li = 0; li < n_hidden; ++li) {
-    a.w[li] = (const f16x8*)((const _Float16*)packed + net.seg[li].offset);
+    a.w[li] = (const bf16x8*)((const __bf16*)packed + 3 * net.seg[2 * li].offset);
     a.b[li] = (const float*)biases[li];
   }
   const bool tail = k_in0 <= 32 * kt0 - 16;  // the last 16-deep step's weights are zero

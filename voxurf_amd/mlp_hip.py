@@ -10,7 +10,8 @@ Precision (`prec` of the kernels):
       every product is formed from three-way BF16 splits of both operands (six BF16
       MFMA products per pair, FP32 accumulation), within 2^-23 relative of the exact
       product, so the results carry FP32 accuracy (the weight gradients too, from
-      operands split once as they are staged in LDS);
+      operands split once as they are staged in LDS); where no gradient follows, all layers
+      in one launch with the same bits (net_logits);
   PREC_F32: the same on FP32 MFMAs (v_mfma_f32_32x32x2f32);
   PREC_BF16 (compute_dtype bfloat16): forward and data-gradient GEMMs as single BF16
       MFMAs with FP32 accumulation, activations stored in BF16; weights, biases,
@@ -48,23 +49,30 @@ def _pad_width(d):
     raise RuntimeError(f"rgbnet input width {d} > 96 is not supported by the MFMA kernels")
 
 
+def _packed_buffer(Ws, prec, st):
+    """Every MFMA operand of one set of weights in one buffer (one vx_mlp_pack_net launch)."""
+    n_hidden = len(Ws) - 1
+    k_in0 = Ws[0].shape[1]
+    total = lib().vx_mlp_pack_net_elems(n_hidden, k_in0)
+    if total < 0:
+        raise RuntimeError("rgbnet shape not supported by the MFMA kernels")
+    parts = 3 if prec == PREC_F32_SPLIT else 1
+    buf = torch.empty(parts * total, dtype=torch.float32 if prec == PREC_F32 else torch.bfloat16,
+                      device=Ws[0].device)
+    w_ptrs = torch.tensor([W.data_ptr() for W in Ws[:-1]], dtype=torch.int64)
+    call("vx_mlp_pack_net", prec, n_hidden, w_ptrs.data_ptr(), k_in0, ptr(buf), st)
+    return buf
+
+
 class Packed:
-    """Every MFMA operand of one set of weights (one vx_mlp_pack_net launch):
-    fwd[li] (layer li, forward) and bwd[li] (layer li transposed, backward)."""
+    """The MFMA operands of one set of weights: fwd[li] (layer li, forward) and bwd[li] (layer
+    li transposed, backward)."""
 
     def __init__(self, Ws, prec, st):
         n_hidden = len(Ws) - 1
-        k_in0 = Ws[0].shape[1]
-        total = lib().vx_mlp_pack_net_elems(n_hidden, k_in0)
-        if total < 0:
-            raise RuntimeError("rgbnet shape not supported by the MFMA kernels")
+        self.buf = _packed_buffer(Ws, prec, st)
         parts = 3 if prec == PREC_F32_SPLIT else 1
-        dev = Ws[0].device
-        self.buf = torch.empty(parts * total, dtype=torch.float32 if prec == PREC_F32 else torch.bfloat16,
-                               device=dev)
-        w_ptrs = torch.tensor([W.data_ptr() for W in Ws[:-1]], dtype=torch.int64)
-        call("vx_mlp_pack_net", prec, n_hidden, w_ptrs.data_ptr(), k_in0, ptr(self.buf), st)
-        kt0 = _pad_width(k_in0) // 32
+        kt0 = _pad_width(Ws[0].shape[1]) // 32
         self.fwd, self.bwd = [], []
         off = 0
         for li in range(n_hidden):
@@ -78,24 +86,15 @@ class Packed:
         self.prec = prec
 
 
-def _addresses(ts):
-    """Host array of device addresses."""
-    return torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64)
-
-
 def net_logits(X, Ws, bs, st, M_dev=None):
-    """logits [M, 3] of padded float32 rows X at split precision without keeping the hidden
+    """The logits [M, 3] of forward_rows at split precision (the same bits) without the hidden
     activations: all layers in one launch, which never writes them (vx_mlp_net_fwd)."""
-    M, dev, n, k_in0 = X.shape[0], X.device, len(Ws) - 1, Ws[0].shape[1]
-    need = lib().vx_mlp_pack_half_bytes(n, k_in0)
-    if need < 0:
-        raise RuntimeError("rgbnet shape not supported by the MFMA kernels")
-    packed = torch.empty(need, dtype=torch.uint8, device=dev)
-    logits = torch.empty((M, 3), dtype=torch.float32, device=dev)
-    w_a, b_a = _addresses(Ws[:-1]), _addresses(bs[:-1])
-    call("vx_mlp_pack_half", n, w_a.data_ptr(), k_in0, ptr(packed), st)
-    call("vx_mlp_net_fwd", n, k_in0, ptr(X), X.shape[1], M, ptr(packed), b_a.data_ptr(),
-         ptr(Ws[-1]), ptr(bs[-1]), ptr(logits), ptr(M_dev), st)
+    M = X.shape[0]
+    logits = torch.empty((M, 3), dtype=torch.float32, device=X.device)
+    packed = _packed_buffer(Ws, PREC_F32_SPLIT, st)
+    b_a = torch.tensor([b.data_ptr() for b in bs[:-1]], dtype=torch.int64)
+    call("vx_mlp_net_fwd", len(Ws) - 1, Ws[0].shape[1], ptr(X), X.shape[1], M, ptr(packed),
+         b_a.data_ptr(), ptr(Ws[-1]), ptr(bs[-1]), ptr(logits), ptr(M_dev), st)
     return logits
 
 
