@@ -239,8 +239,9 @@ int vx_sdf_query(const float* sdf, const int64_t* geom, const float* box, float 
 
 /* Occupancy of a MaskCache: which bricks and blocks of its grid hold a sample that could pass
  * (vx_maskcache_occupancy_bytes bytes, 8-byte aligned; -1: bad geometry).  The _occ forms of
- * the two entries above take it (or NULL) and give the same flags, jumping over what is
- * clear; it must be that of the same mc, mc_geom and mc_params. */
+ * the two entries above take it (or NULL, as the two entries above: a wavefront a ray that
+ * looks every sample up) and give the same flags, a thread a ray jumping over what is clear;
+ * it must be that of the same mc, mc_geom and mc_params. */
 int64_t vx_maskcache_occupancy_bytes(const int64_t* mc_geom);
 int vx_maskcache_occupancy(const float* mc, const int64_t* mc_geom, const float* mc_params,
                            void* occ, void* stream);

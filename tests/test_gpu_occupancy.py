@@ -44,7 +44,8 @@ def _density(kind, shape, g):
                                   dict(thres=0.5, ratio=0.3), dict(thres=0.0), dict(thres=1.0),
                                   dict(box=((-0.4, -0.3, -0.2), (0.5, 0.9, 0.6))),
                                   dict(box=((-3.0, -2.0, -1.5), (1.2, 4.0, 2.0)))])
-def test_occupancy_gives_the_same_hits(dev, kind, shape, ks, opts):
+def test_occupancy_gives_the_same_hits(dev, kind, shape, ks, opts, monkeypatch):
+    monkeypatch.setattr(vr, "OCC_RAYS", 0)   # the walk with occupancy bits for any number of rays
     g = torch.Generator().manual_seed(sum(shape) + len(kind))
     box = opts.get("box", ((-1.0, -1.0, -1.0), (1.0, 1.0, 1.0)))
     mc = MaskCache(density=_density(kind, shape, g)[None, None], ks=ks, xyz_min=box[0],
@@ -95,3 +96,44 @@ def test_occupancy_bytes(dev):
     geom = torch.tensor([1, 700, 700, 700, 1, 490000, 700, 1], dtype=torch.int64)
     assert 0 < lib().vx_maskcache_occupancy_bytes(geom.data_ptr()) <= 9 << 17
     assert lib().vx_maskcache_occupancy_bytes(None) == -1
+
+
+def test_few_rays_take_no_occupancy(dev, monkeypatch):
+    """Small calls look every sample up, a wavefront a ray, without a pass over the cache's grid;
+    the flags on both sides of the line are the same."""
+    made = []
+    make = vr._occupancy
+    monkeypatch.setattr(vr, "_occupancy", lambda *a: made.append(1) or make(*a))
+    g = torch.Generator().manual_seed(5)
+    mc = MaskCache(density=_density("shell", (64, 64, 64), g)[None, None], ks=3, xyz_min=[-1.0] * 3,
+                   xyz_max=[1.0] * 3, act_shift=-4.6, voxel_size_ratio=1.0).to(dev)
+    o, d, _ = scene.rays(40000, seed=3, jitter=0.4)
+    o, d = o.to(dev).contiguous(), d.to(dev).contiguous()
+    hit = vr.hit_coarse_geo(mc, [-1.0] * 3, [1.0] * 3, o, d, 0.0, 1.0 / 64)
+    assert made == [1]
+    for n in (0, 1, 1000, 8192):
+        few = vr.hit_coarse_geo(mc, [-1.0] * 3, [1.0] * 3, o[:n], d[:n], 0.0, 1.0 / 64)
+        assert torch.equal(few, hit[:n])
+    assert made == [1]
+
+    class Model:
+        mask_cache, xyz_min, xyz_max, voxel_size = mc, [-1.0] * 3, [1.0] * 3, 1.0 / 32
+
+    c2w = torch.tensor([[1.0, 0, 0, 0], [0, 0, -1, -3.0], [0, 1, 0, 0.1]])
+    K = [[60.0, 0, 32], [0, 60.0, 24], [0, 0, 1]]
+    img = torch.rand((48, 64, 3), generator=g).to(dev)
+
+    def views(pixels):
+        monkeypatch.setattr(vr, "OCC_PIXELS", pixels)
+        return vr.get_training_rays_in_maskcache_sampling(
+            [img, img[:, :9]], [c2w] * 2, [(48, 64), (48, 9)], [K] * 2, False, False, False, False,
+            Model, dict(near=0.0, stepsize=0.5))
+
+    few = views(vr.OCC_PIXELS)
+    assert made == [1]
+    # one of the two views past the line, then both: the bits are made once a call
+    for pixels, calls in ((1000, 2), (100, 3)):
+        some = views(pixels)
+        assert len(made) == calls and some[4] == few[4]
+        assert all(torch.equal(a, b) for a, b in zip(some[:4], few[:4]))
+    assert 0 < few[4][0] < 48 * 64

@@ -5,7 +5,8 @@
 // hit_coarse_geo (lib/voxurf_fine.py:579-591) samples every step of every ray, then looks
 // up the MaskCache at every in-box point and scatters the hits; here one thread walks one
 // ray, jumps over the bricks of the coarse grid in which no sample can pass, and stops at the
-// first step that passes the mask.
+// first step that passes the mask; few rays take a wavefront each, 64 steps at a time, until
+// one passes.
 // get_training_rays_in_maskcache_sampling (lib/voxurf_fine.py:1127-1164) becomes, per
 // view: hit flags straight from the camera (no ray arrays), an inclusive scan, and a
 // compaction that rebuilds the kept rays with the same arithmetic and writes them in
@@ -118,7 +119,7 @@ __global__ void __launch_bounds__(256) k_ndc_rays(int64_t n, float c0, float c1,
 // from inverting alpha(d) = thres in double with a margin far above the float formula's
 // error, so that the float test itself decides between them and only there.
 struct Occupancy {
-  const uint32_t* bits;      // brick has a block that may pass; nullptr: look everything up
+  const uint32_t* bits;      // brick has a block that may pass; nullptr: not known
   const uint32_t* near;      // it or one of the 26 around it has
   const uint64_t* blocks;    // its blocks: bit 16 x + 4 y + z
   int shift, bx, by, bz;     // bricks per axis
@@ -188,8 +189,60 @@ __global__ void __launch_bounds__(256) k_occupancy_near(Occupancy oc, const uint
 }
 
 // Does any in-box sample of the ray pass the MaskCache?  Samples exactly as
-// sample_pts_on_rays; with occupancy bits, a sample is looked up only where its block's bit
-// is set or the block is in doubt: the walk follows the straight line through the cache's
+// sample_pts_on_rays.  The wave looks 64 at a time up and leaves at the first chunk that
+// holds a passing one.
+__device__ __forceinline__ bool wave_hits(const FusedGeom& G, const float* o, const float* d,
+                                          int lane) {
+  float start[3], dir[3];
+  int64_t n;
+  ray_setup(G, o, d, start, dir, n);
+  for (int64_t base = 0; base < n; base += 64) {
+    const int64_t s = base + lane;
+    bool pass = false;
+    if (s < n) {
+      float q[3];
+      if (!sample_point<float>(start, dir, G.mn, G.mx, G.stepdist, s, q[0], q[1], q[2]))
+        pass = maskcache_pass(G, q);
+    }
+    if (__ballot(pass)) return true;
+  }
+  return false;
+}
+
+// One wavefront per ray: hit (bool bytes) and/or flag (int64 0/1) per ray.
+__global__ void __launch_bounds__(256) k_hit_rays_wave(FusedGeom G, const float* __restrict__ rays_o,
+                                                       const float* __restrict__ rays_d,
+                                                       int64_t n_rays, uint8_t* __restrict__ hit,
+                                                       int64_t* __restrict__ flag) {
+  const int lane = threadIdx.x & 63;
+  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); r < n_rays;
+       r += waves) {
+    const bool h = wave_hits(G, rays_o + 3 * r, rays_d + 3 * r, lane);
+    if (lane == 0) {
+      if (hit) hit[r] = h;
+      if (flag) flag[r] = h;
+    }
+  }
+}
+
+// The same for a view, each pixel's ray made by every lane of its wave (a few dozen flops,
+// cheaper than a broadcast).
+__global__ void __launch_bounds__(256) k_hit_camera_wave(FusedGeom G, Camera c,
+                                                         int64_t* __restrict__ flag) {
+  const int lane = threadIdx.x & 63;
+  const int64_t n = (int64_t)c.H * c.W;
+  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  for (int64_t p = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); p < n; p += waves) {
+    float o[3], d[3], v[3];
+    camera_ray(c, (int)(p / c.W), (int)(p % c.W), o, d, v);
+    const bool h = wave_hits(G, o, d, lane);
+    if (lane == 0) flag[p] = h;
+  }
+}
+
+// The same question with occupancy bits, a thread a ray: a sample is looked up only where its
+// block's bit is set or the block is in doubt: the walk follows the straight line through the cache's
 // grid, which a sample's own index is off by less than `margin` cells, and from a sample
 // inside a clear brick or block by more than that it goes on with the first one that is not.
 // A lookup on that line decides too, unless the margin could change the answer: then the
@@ -203,7 +256,7 @@ __device__ __forceinline__ bool ray_hits(const FusedGeom& G, const Occupancy& oc
   // index of the line at the first step, cells per step, steps per cell; the margin at the
   // side where it leaves a box
   float p0[3], rate[3], inv[3], far[3];
-  bool line = bits && n < (1 << 24);  // (float) s is exact
+  bool line = n < (1 << 24);  // (float) s is exact
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const float cells = (float)(size[a] - 1) / (G.mc_mx[a] - G.mc_mn[a]);
@@ -317,7 +370,7 @@ __global__ void __launch_bounds__(256) k_hit_rays(FusedGeom G, Occupancy oc,
                                                   uint8_t* __restrict__ hit,
                                                   int64_t* __restrict__ flag) {
   const int words = (oc.bx * oc.by * oc.bz + 31) >> 5;
-  const uint32_t* bits = oc.bits ? occ_to_lds(oc.bits, words, 0) : nullptr;
+  const uint32_t* bits = occ_to_lds(oc.bits, words, 0);
   __syncthreads();
   for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_rays;
        r += (int64_t)gridDim.x * blockDim.x) {
@@ -344,8 +397,8 @@ __global__ void __launch_bounds__(256) k_hit_rays(FusedGeom G, Occupancy oc,
 __global__ void __launch_bounds__(256) k_hit_camera(FusedGeom G, Occupancy oc, Camera c,
                                                     int64_t* __restrict__ flag) {
   const int words = (oc.bx * oc.by * oc.bz + 31) >> 5;
-  const uint32_t* bits = oc.bits ? occ_to_lds(oc.bits, words, 0) : nullptr;
-  const uint32_t* near = oc.bits ? occ_to_lds(oc.near, words, words) : nullptr;
+  const uint32_t* bits = occ_to_lds(oc.bits, words, 0);
+  const uint32_t* near = occ_to_lds(oc.near, words, words);
   __syncthreads();
   const int tw = (c.W + 7) >> 3, th = (c.H + 7) >> 3, lane = threadIdx.x & 63;
   const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
@@ -358,7 +411,7 @@ __global__ void __launch_bounds__(256) k_hit_camera(FusedGeom G, Occupancy oc, C
     camera_ray(c, min(row, c.H - 1), min(col, c.W - 1), o, d, v);
     int64_t n, s0 = 0;
     ray_setup(G, o, d, start, dir, n);
-    if (near && oc.inner && !c.ndc) {
+    if (oc.inner && !c.ndc) {
       // distances from the camera at which this ray's samples begin and end
       float t0 = 0.f, dev = 0.f, mid[3];
 #pragma unroll
@@ -537,7 +590,7 @@ static Occupancy occupancy_of(const FusedGeom& G, const void* occ) {
 
 // LDS of `arrays` copies of the bits.
 static size_t occ_lds_bytes(const Occupancy& oc, int arrays) {
-  return oc.bits ? (size_t)cdiv((int64_t)oc.bx * oc.by * oc.bz, 32) * 4 * arrays : 0;
+  return (size_t)cdiv((int64_t)oc.bx * oc.by * oc.bz, 32) * 4 * arrays;
 }
 
 extern "C" {
@@ -597,8 +650,12 @@ int vx_hit_coarse_geo_occ(const float* rays_o, const float* rays_d, int64_t n_ra
   if (n_rays == 0) return VX_OK;
   VX_CHECK_ARG(hit || flag, "hit_coarse_geo: no output");
   const Occupancy oc = occupancy_of(G, occ);
-  k_hit_rays<<<grid_for(n_rays, 256), 256, occ_lds_bytes(oc, 1), (hipStream_t)stream>>>(
-      G, oc, rays_o, rays_d, n_rays, hit, flag);
+  if (oc.bits)
+    k_hit_rays<<<grid_for(n_rays, 256), 256, occ_lds_bytes(oc, 1), (hipStream_t)stream>>>(
+        G, oc, rays_o, rays_d, n_rays, hit, flag);
+  else
+    k_hit_rays_wave<<<grid_for(n_rays, 4, 1 << 16), 256, 0, (hipStream_t)stream>>>(
+        G, rays_o, rays_d, n_rays, hit, flag);
   return launch_status("hit_coarse_geo");
 }
 
@@ -619,6 +676,10 @@ int vx_view_hit_coarse_geo_occ(const float* cam, const float* box, const float* 
   const int64_t n = (int64_t)c.H * c.W;
   if (n == 0) return VX_OK;
   const Occupancy oc = occupancy_of(G, occ);
+  if (!oc.bits) {
+    k_hit_camera_wave<<<grid_for(n, 4, 1 << 16), 256, 0, (hipStream_t)stream>>>(G, c, flag);
+    return launch_status("view_hit_coarse_geo");
+  }
   const int64_t tiles = cdiv(c.W, 8) * cdiv(c.H, 8);
   VX_CHECK_ARG(tiles < ((int64_t)1 << 32), "hit_coarse_geo: view too large");
   // a tile per wave: the walks along the object's outline are ten times the others', and a

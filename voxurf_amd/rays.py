@@ -92,6 +92,17 @@ def _prefilter_args(mask_cache, xyz_min, xyz_max, near, stepdist):
     return box, params, maskcache_args(mask_cache)
 
 
+# Rays of a call, and pixels of a view, past which the walks with occupancy bits are taken.  They
+# need the bits (a pass over the cache's grid: 85 us for 256^3) and a thread a ray, whose chain
+# of steps is as long for one ray as for many; a wavefront a ray that looks every sample up is
+# through after a few chunks of 64.  Whole calls in us, wavefront / bits, for a shell in a 100^3
+# cache at steps of a voxel: 8192 rays 21 / 58, 32768 42 / 61, 65536 75 / 61; views of 200^2
+# pixels 127 / 342, 400^2 292 / 419, 460^2 364 / 447, 512^2 452 / 346 (256^3: 835 / 741 at
+# 460^2; an empty cache sooner: 218 / 147 at 300^2, but no step in it is looked up).
+OCC_RAYS = 1 << 15
+OCC_PIXELS = 200000
+
+
 def _occupancy(mask_cache, mc):
     """The MaskCache's occupancy (vx_maskcache_occupancy) for one call's walks."""
     need = lib().vx_maskcache_occupancy_bytes(mc[1])
@@ -112,7 +123,7 @@ def hit_coarse_geo(mask_cache, xyz_min, xyz_max, rays_o, rays_d, near, stepdist)
         raise RuntimeError("hit_coarse_geo: rays_o and rays_d differ in shape")
     box, params, mc = _prefilter_args(mask_cache, xyz_min, xyz_max, near, stepdist)
     hit = torch.empty(o.shape[0], dtype=torch.bool, device=o.device)
-    occ = _occupancy(mask_cache, mc)
+    occ = _occupancy(mask_cache, mc) if o.shape[0] > OCC_RAYS else None
     call("vx_hit_coarse_geo_occ", ptr(o), ptr(d), o.shape[0], box.data_ptr(), params.data_ptr(),
          *mc, ptr(occ), ptr(hit), None, stream_of(o))
     return hit.reshape(shape)
@@ -140,7 +151,7 @@ def get_training_rays_in_maskcache_sampling(rgb_tr_ori, train_poses, HW, Ks, ndc
     rays_o_tr = torch.empty_like(rgb_tr)
     rays_d_tr = torch.empty_like(rgb_tr)
     viewdirs_tr = torch.empty_like(rgb_tr)
-    occ = _occupancy(model.mask_cache, mc)
+    occ = None
     imsz = []
     top = 0
     st = stream_of(rgb_tr)
@@ -149,8 +160,11 @@ def get_training_rays_in_maskcache_sampling(rgb_tr_ori, train_poses, HW, Ks, ndc
         cam = camera_params(H, W, K, c2w, inverse_y, flip_x, flip_y, "center", ndc)
         n = H * W
         flag = torch.empty(n, dtype=torch.int64, device=dev)
+        large = n > OCC_PIXELS
+        if large and occ is None:
+            occ = _occupancy(model.mask_cache, mc)
         call("vx_view_hit_coarse_geo_occ", cam.data_ptr(), box.data_ptr(), params.data_ptr(), *mc,
-             ptr(occ), ptr(flag), st)
+             ptr(occ) if large else None, ptr(flag), st)
         incl = torch.empty_like(flag)
         ws = torch.empty(max(1, lib().vx_scan_workspace_elems(n)), dtype=torch.int64, device=dev)
         call("vx_inclusive_scan_i64", ptr(flag), ptr(incl), n, ptr(ws), st)
