@@ -50,6 +50,39 @@ def test_groups_match_per_point(dev, shape, kind):
     assert torch.equal(torch.nan_to_num(v, nan=77.0), torch.nan_to_num(rv, nan=77.0))
 
 
+def test_a_dense_field_is_no_slower(dev):
+    """Noise, every point of which is listed, on a lattice of few workgroups: writing its mesh takes
+    at most twice the per-point passes' time (one workgroup a list took ten times it)."""
+    u = (torch.rand((64, 64, 64), generator=torch.Generator().manual_seed(0)) * 2 - 1).to(dev)
+    n, st = u.numel(), stream_of(u)
+    count, edges = (torch.from_numpy(t).to(dev) for t in mesh.mc_tables_host())
+    cnt = torch.empty((2, n), dtype=torch.int64, device=dev)
+    call("vx_mc_count", ptr(u), 64, 64, 64, 0.0, ptr(count), ptr(edges), ptr(cnt[0]), ptr(cnt[1]), st)
+    incl = cnt.cumsum(1)
+    nv, nf = incl[:, -1].tolist()
+    ws = torch.empty(lib().vx_mc_workspace_bytes(64, 64, 64) // 8, dtype=torch.int64, device=dev)
+    tot = torch.empty(2, dtype=torch.int64, device=dev)
+    call("vx_mc_classify", ptr(u), 64, 64, 64, 0.0, ptr(count), ptr(ws), ptr(tot), st)
+    assert tot.tolist() == [nv, nf]
+    verts = torch.empty((nv, 3), dtype=torch.float64, device=dev)
+    faces = torch.empty((nf, 3), dtype=torch.int64, device=dev)
+    forms = [lambda: call("vx_mc_write", ptr(u), 64, 64, 64, 0.0, ptr(count), ptr(edges), ptr(ws), nv,
+                          nf, None, ptr(verts), ptr(faces), st),
+             lambda: call("vx_mc_emit", ptr(u), 64, 64, 64, 0.0, ptr(count), ptr(edges), ptr(incl[0]),
+                          ptr(incl[1]), None, ptr(verts), ptr(faces), st)]
+    best = [1e9, 1e9]
+    for _ in range(10):
+        for k, form in enumerate(forms):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                form()
+            b.record()
+            torch.cuda.synchronize()
+            best[k] = min(best[k], a.elapsed_time(b))
+    assert best[0] <= 2 * best[1], best
+
+
 def test_bad_sizes_are_refused(dev):
     for shape in [(0, 2, 2), (65536, 1, 1)]:
         with pytest.raises(VoxhipError):

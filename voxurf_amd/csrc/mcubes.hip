@@ -598,7 +598,7 @@ struct McWorld {
 // A block's groups once more: their points that own a vertex or whose cube is cut are listed
 // in LDS in point order (a group is a row's 64 points, of which the surface takes one or two),
 // then a lane takes a point each.  With a wave per group and a lane per point of it the waves
-// ran nearly empty: 797 us for the 900 k vertices of a 512^3 mesh.
+// ran nearly empty: 797 us for the 381 k vertices of a 512^3 mesh, 172 so.
 __global__ void __launch_bounds__(kMcThreads) k_mc_write(McArgs a, McGroups g, McWorld wd,
                                                          double* __restrict__ verts,
                                                          int64_t* __restrict__ faces) {
@@ -645,7 +645,7 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_write(McArgs a, McGroups g, M
   __syncthreads();
   const int64_t sx = (int64_t)a.ny * a.nz, sy = a.nz;
   const int nn[3] = {a.nx, a.ny, a.nz};
-  for (int p = threadIdx.x; p < total; p += kMcThreads) {
+  for (int p = blockIdx.y * kMcThreads + threadIdx.x; p < total; p += gridDim.y * kMcThreads) {
     const uint32_t en = list[p];
     const int bit = en & 63, cfg = en >> 13 & 255;
     const int64_t q = first + (en >> 6 & 127);
@@ -861,8 +861,13 @@ int vx_mc_write(const float* u, int nx, int ny, int nz, float iso, const int8_t*
       wd.bmin[i] = (double)(float)bounds[i];
       wd.ext[i] = (double)((float)bounds[3 + i] - (float)bounds[i]);
     }
-  k_mc_write<<<(unsigned)blocks, kMcThreads, 0, (hipStream_t)stream>>>(a, g, wd, verts,
-                                                                      faces);
+  // about n_faces / 2 points are listed, which workgroups share where that is more than a pass
+  // of them each: with one a list, a 64^3 lattice of noise ran in 32 (535 us the call, 79 with
+  // 32 shares, 92 with 16; 128^3, in 256: 584, 305 and 284).  Each makes the whole list.
+  const int64_t passes = cdiv(n_faces, 2 * blocks * kMcThreads), most = blocks < 64 ? 32 : 16;
+  const unsigned shares = (unsigned)(passes < 1 ? 1 : (passes > most ? most : passes));
+  k_mc_write<<<dim3((unsigned)blocks, shares), kMcThreads, 0, (hipStream_t)stream>>>(a, g, wd, verts,
+                                                                                    faces);
   return launch_status("mc_write");
 }
 
