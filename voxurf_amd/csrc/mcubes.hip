@@ -659,7 +659,7 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_write(McArgs a, McGroups g, M
     };
     // the number of the vertex on edge `ax` of the point at (i + di, j + dj, k + dk)
     auto vertex = [&](int di, int dj, int dk, int ax) {
-      uint64_t e[3], nb = 0, ni = 0, nj = 0;
+      uint64_t e[3], nb = 0, ni = 0;
 #pragma unroll
       for (int x = 0; x < 2; ++x)
 #pragma unroll
@@ -668,7 +668,6 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_write(McArgs a, McGroups g, M
             mc_edges(a, m, i, j, x, y, e);
             nb = m.n[x][y];
             ni = m.n[x + 1][y];
-            nj = m.n[x][y + 1];
           }
       const int64_t gq = ((int64_t)(i + di) * a.ny + (j + dj)) * g.words + w;
       if (bit + dk < 64) {
@@ -680,8 +679,8 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_write(McArgs a, McGroups g, M
       }
       // the first point of the row's next word: no point of its group comes before it
       int64_t v = first_vertex(gq + 1);
+      // (nor a z edge: those of this cube start in its own word)
       if (ax > 0 && i + di + 1 < a.nx) v += (nb ^ ni) & 1;
-      if (ax > 1 && j + dj + 1 < a.ny) v += (nb ^ nj) & 1;
       return v;
     };
     uint64_t own[3];
