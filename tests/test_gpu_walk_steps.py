@@ -1,4 +1,5 @@
-"""The transmittance walk of alpha2weight (eight steps at a time) against the sequential
+"""The transmittance walk of alpha2weight (eight steps at a time, a rest of up to three by
+itself) against the sequential
 recurrence T = float(double(T) (1 - double(alpha))), to the bit: segments around eight and 64
 samples, walks that end at every step of an eight, a NaN."""
 import pytest
@@ -10,14 +11,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-def test_walk_ends_at_every_step(dev, dtype):
-    """Ray r of length r: alphas that bring T below 1e-3 at step r - 3 or never, and a NaN."""
+@pytest.mark.parametrize("back", [3, 1, 2])
+def test_walk_ends_at_every_step(dev, dtype, back):
+    """Ray r of length r: alphas that bring T below 1e-3 at step r - back or never, and a NaN."""
     g = torch.Generator().manual_seed(3)
     alpha, ids = [], []
     for r in range(150):
         a = torch.rand(r, generator=g, dtype=torch.float64) * 0.02
         if r > 3 and r % 2:
-            a[r - 3] = 0.9999
+            a[r - back] = 0.9999
         if r == 77:
             a[20] = float("nan")
         alpha.append(a)

@@ -455,7 +455,8 @@ __global__ void __launch_bounds__(256) k_a2w_scan(const T* __restrict__ alpha,
       const int cnt = (int)((ie - base) < 64 ? (ie - base) : 64);
       float myT = 1.f;
       bool done = false;
-      for (int k0 = 0; k0 < cnt && !done; k0 += 8) {
+      int k0 = 0;
+      for (; k0 + 3 < cnt && !done; k0 += 8) {
         // eight steps (past the segment's end: through = 1), and one look at whether the
         // walk ended in them
         const float T0 = Tc;
@@ -474,6 +475,13 @@ __global__ void __launch_bounds__(256) k_a2w_scan(const T* __restrict__ alpha,
             stop = base + k + 1;
           }
         }
+      }
+      // a rest of one to three by itself: eight steps for rays of a single sample took 32 us for
+      // 100,000 of them, one 25
+      for (; k0 < cnt && !done; ++k0) {
+        if (lane == k0) myT = Tc;
+        done = walk_step(Tc, through, k0);
+        if (done) stop = base + k0 + 1;
       }
       if (i < stop && i < ie) {
         Tt[i] = (T)myT;
