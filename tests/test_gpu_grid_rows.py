@@ -65,10 +65,11 @@ def test_lookup_and_scatter(dev, C, pad, n, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("n", [1, 2, 64, 65, 1000])
+@pytest.mark.parametrize("n", [1, 2, 64, 65, 255, 256, 257, 321, 1000])
 @pytest.mark.parametrize("which", ["both", "sdf", "grad"])
 def test_sdf_scatter_runs(dev, n, which, dtype):
-    """With and without (zero) neighbour-value gradients: the plain form and the runs'."""
+    """With and without (zero) neighbour-value gradients: the plain form and the runs' (from 256
+    samples on)."""
     g = torch.Generator().manual_seed(n)
     shape = (1, 1, 13, 9, 11)
     mn, mx = torch.full((3,), -1.0).to(dev, dtype), torch.full((3,), 1.0).to(dev, dtype)
