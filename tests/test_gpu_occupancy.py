@@ -91,6 +91,42 @@ def test_view_gives_the_same_hits(dev, H, W, focal, kind, eye):
         assert torch.equal(flag != 0, want)
 
 
+@pytest.mark.parametrize("dist", [30.0, 1e3, 4.9e3, 4e4, 3e5])
+@pytest.mark.parametrize("stepdist", [1.0 / 200, 0.05, 0.31])
+@pytest.mark.parametrize("kind", ["shell", "sparse", "grains"])
+def test_view_from_very_far(dev, dist, stepdist, kind):
+    """Every pixel's flag from cameras so far off that their rays' coordinates are rounded to a
+    good part of a cell, or to several; tiles of a fifth of a brick and of five."""
+    import numpy as np
+    g = torch.Generator().manual_seed(17)
+    shape = (200, 190, 201)
+    if kind == "grains":     # lone lattice points: bricks that few rays meet
+        dens = torch.where(torch.rand(shape, generator=g) < 2e-4, 5.0, -20.0)
+    else:
+        dens = _density(kind, shape, g)
+    mc = MaskCache(density=dens[None, None], ks=1, xyz_min=[-1.0, -1.1, -1.0],
+                   xyz_max=[1.0, 1.0, 1.2], act_shift=-4.6, voxel_size_ratio=1.0).to(dev)
+    box, params, args = vr._prefilter_args(mc, [-1.0] * 3, [1.0] * 3, 0.0, stepdist)
+    occ = vr._occupancy(mc, args)
+    H = W = 240
+    for way, zoom in (((0.0, -1.0, 0.1), 1000.0), ((0.5, 0.6, -0.7), 1000.0), ((-1.0, 0.0, 0.003), 300.0),
+                      ((0.31, -0.9, 0.2), 40.0)):
+        focal = zoom * dist
+        K = np.array([[focal, 0, W / 2], [0, focal, H / 2], [0, 0, 1]])
+        e = torch.tensor(way) / torch.tensor(way).norm() * dist
+        fwd = -e / e.norm()
+        right = torch.linalg.cross(fwd, torch.tensor([0.0, 0.0, 1.0]))
+        right = right / right.norm()
+        c2w = torch.stack([right, torch.linalg.cross(right, fwd), -fwd, e], 1)
+        cam = vr.camera_params(H, W, K, c2w, False, False, False, "center", False)
+        flag, want = (torch.empty(H * W, dtype=torch.int64, device=dev) for _ in range(2))
+        call("vx_view_hit_coarse_geo_occ", cam.data_ptr(), box.data_ptr(), params.data_ptr(), *args,
+             ptr(occ), ptr(flag), stream_of(flag))
+        call("vx_view_hit_coarse_geo", cam.data_ptr(), box.data_ptr(), params.data_ptr(), *args,
+             ptr(want), stream_of(flag))
+        assert torch.equal(flag, want), int((flag != want).sum())
+
+
 def test_occupancy_bytes(dev):
     # bricks grow until their bits fit the LDS copy: at most 2^17 of them
     geom = torch.tensor([1, 700, 700, 700, 1, 490000, 700, 1], dtype=torch.int64)
