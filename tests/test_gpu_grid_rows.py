@@ -193,3 +193,20 @@ def test_sdf_query(dev, tile, origin, res):
     # (outside the box the clamped neighbours coincide: no direction, in either form)
     want = rg / (rg.norm(dim=-1, keepdim=True) + 1e-5)
     assert torch.allclose(n, want, rtol=1e-6, atol=1e-7, equal_nan=True)
+
+
+def test_sdf_query_forms(dev):
+    """A tile given as a float (as arange takes it), origins in tensors, an empty tile, and a
+    default device other than the host's."""
+    import dataclasses
+    cfg = dataclasses.replace(scene.FINE, R=24, feat_dim=3)
+    sc = serve.ResidentScene(cfg, scene.sdf_grid(24), scene.feature_grid(24, 3),
+                             scene.mlp_params(cfg.mlp_in, 192, 4), device=dev)
+    want = sc.sdf_query(30, (1, 2, 3), 5)
+    forms = [((1, 2, 3), 5.0), (torch.tensor([1, 2, 3]), 5), (torch.tensor([1.0, 2.0, 3.0]).to(dev), 4.5)]
+    for origin, tile in forms:
+        assert all(torch.equal(a, b) for a, b in zip(sc.sdf_query(30, origin, tile), want))
+    with torch.device(dev):
+        assert all(torch.equal(a, b) for a, b in zip(sc.sdf_query(30, (1, 2, 3), 5), want))
+    s, n = sc.sdf_query(30, (1, 2, 3), 0)
+    assert s.shape == (0,) and n.shape == (0, 3)

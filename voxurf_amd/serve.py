@@ -23,6 +23,7 @@ import queue
 import threading
 import time
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -170,12 +171,16 @@ class ResidentScene:
     def sdf_query(self, res, tile_origin, tile=64):
         """SDF and unit normal at a tile of the res^3 lattice over the bbox
         (x_i = -1 + 2 i / (res - 1)): points [tile^3, 3] -> (sdf [P], normal [P, 3])."""
-        origin = torch.tensor([float(v) for v in tile_origin], dtype=torch.float32)
+        i0, j0, k0 = tile_origin  # three of them: the kernel's call reads that many
+        origin = np.array([float(i0), float(j0), float(k0)], dtype=np.float32)
+        tile = math.ceil(tile)    # as many points as arange(tile) has
+        if tile < 0:
+            raise ValueError("sdf_query: negative tile")
         n = tile ** 3
         sdf = torch.empty(n, dtype=torch.float32, device=self.dev)
         normal = torch.empty((n, 3), dtype=torch.float32, device=self.dev)
         call("vx_sdf_query", ptr(self.sdf), self.sdf_geom.data_ptr(), self.box.data_ptr(),
-             float(self.cfg.voxel_size), float(res), origin.data_ptr(), int(tile), ptr(sdf),
+             float(self.cfg.voxel_size), float(res), origin.ctypes.data, tile, ptr(sdf),
              ptr(normal), stream_of(self.sdf))
         return sdf, normal
 
