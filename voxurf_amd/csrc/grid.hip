@@ -938,12 +938,13 @@ int vx_total_variation_add_grad_new(int dtype, const void* param, void* grad, co
 
 int vx_sdf_query(const float* sdf, const int64_t* geom, const float* box, float voxel_size,
                  float res, const float* origin, int tile, float* out, float* normal, void* stream) {
-  VX_CHECK_ARG(sdf && geom && box && origin && out && normal, "sdf_query: missing argument");
+  VX_CHECK_ARG(sdf && geom && box && origin, "sdf_query: missing argument");
   QueryArgs a;
   if (int st = make_desc(geom, a.g)) return st;
   VX_CHECK_ARG(a.g.C == 1, "sdf_query: the SDF grid must have one channel");
   VX_CHECK_ARG(tile >= 0 && tile <= 65535, "sdf_query: bad tile size");
   if (tile == 0) return VX_OK;
+  VX_CHECK_ARG(out && normal, "sdf_query: missing output");
   a.sdf = sdf;
   for (int i = 0; i < 3; ++i) {
     a.mn[i] = box[i];
