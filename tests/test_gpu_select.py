@@ -49,3 +49,23 @@ def test_other_forms_are_indexed(dev):
     assert torch.equal(x.grad, mask.float()) and y.grad is None
     with torch.no_grad():
         assert not select_rows(mask, x)[0].requires_grad
+
+
+def test_differentiated_twice_and_forward(dev):
+    """The gradient's gradient and the forward-mode derivative are indexing's."""
+    import torch.autograd.forward_ad as fwd
+    g = torch.Generator(device=dev).manual_seed(2)
+    mask = torch.rand(5000, generator=g, device=dev) < 0.3
+    x, y, t = (torch.randn(5000, 3, generator=g, device=dev, requires_grad=True) for _ in range(3))
+    res = []
+    for pick in (select_rows, lambda m, *a: tuple(v[m] for v in a)):
+        a, b = pick(mask, x, y)
+        first = torch.autograd.grad((a.pow(3) * b).sum(), (x, y), create_graph=True)
+        second = torch.autograd.grad((first[0] * y + first[1].pow(2)).sum(), (x, y))
+        with fwd.dual_level():
+            a, b = pick(mask, fwd.make_dual(x.detach(), t.detach()), y.detach())
+            a, b = fwd.unpack_dual(a), fwd.unpack_dual(b)
+        res.append([*first, *second, a.primal, a.tangent, b.primal])
+        assert b.tangent is None
+    for u, v in zip(*res):
+        assert torch.equal(u, v)

@@ -12,7 +12,10 @@ same quantities with F.grid_sample, elementwise torch ops and torch_scatter:
   select_rows       the x[mask] compactions between the stages
   SegmentSum        torch_scatter.segment_coo(reduce='sum') at lib/voxurf_fine.py:753-777
 """
+import ctypes
+
 import torch
+import torch.autograd.forward_ad as fwd
 
 from . import render_utils_cuda as ru
 from ._lib import call, dtype_code, lib, ptr, stream_of
@@ -231,56 +234,85 @@ def _row_words(t):
     return t.element_size() * (t.numel() // max(t.shape[0], 1)) // 4
 
 
-def _copy_rows(mask, offsets, src, dst, transpose):
-    s, d = (torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64) for ts in (src, dst))
-    w = torch.tensor([_row_words(t) for t in (dst if transpose else src)], dtype=torch.int32)
-    call("vx_select_rows", ptr(mask), mask.shape[0], ptr(offsets), len(src), s.data_ptr(),
-         d.data_ptr(), w.data_ptr(), transpose, stream_of(mask))
-
-
-class _SelectRows(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, mask, *arrays):
-        n = mask.shape[0]
-        offsets = torch.empty(lib().vx_select_blocks(n), dtype=torch.int32, device=mask.device)
-        total = torch.empty(1, dtype=torch.int64, device=mask.device)
-        call("vx_select_count", ptr(mask), n, ptr(offsets), ptr(total), stream_of(mask))
+def _moved_rows(mask, offsets, m, spread, arrays):
+    """The selected rows of each array (spread 0), or its rows spread over the mask (1)."""
+    n = mask.shape[0]
+    out = [a.new_empty((n if spread else m, *a.shape[1:])) for a in arrays]
+    if spread or m:
         src = [a.contiguous() for a in arrays]
-        m = int(total.item())
-        out = [torch.empty((m, *a.shape[1:]), dtype=a.dtype, device=a.device) for a in src]
-        if m:
-            _copy_rows(mask, offsets, src, out, 0)
-        ctx.mark_non_differentiable(*[o for o, g in zip(out, ctx.needs_input_grad[1:]) if not g])
+        k = len(src)
+        # host arrays: k sources, k destinations, k row lengths
+        s, d = (ctypes.c_int64 * k)(*map(ptr, src)), (ctypes.c_int64 * k)(*map(ptr, out))
+        w = (ctypes.c_int * k)(*map(_row_words, out))
+        call("vx_select_rows", ptr(mask), n, ptr(offsets), k, s, d, w, spread, stream_of(mask))
+    return out
+
+
+def _each_given(fn, ts):
+    """fn of those of ts that are given, None for the others."""
+    given = [t for t in ts if t is not None]
+    out = iter(fn(*given) if given else ())
+    return tuple(None if t is None else next(out) for t in ts)
+
+
+def _carries(t):
+    """Whether a derivative follows t: a gradient to come or a tangent beside it."""
+    return t.requires_grad or fwd.unpack_dual(t).tangent is not None
+
+
+class _MoveRows(torch.autograd.Function):
+    """Rows under a mask (offsets: vx_select_count's), m of them selected.  spread 0: the selected
+    rows of each array; 1, the adjoint: rows where mask selects, zeros elsewhere.  carries: the
+    arrays that a derivative follows."""
+
+    @staticmethod
+    def forward(ctx, mask, offsets, m, spread, carries, *arrays):
+        out = _moved_rows(mask, offsets, m, spread, arrays)
+        ctx.mark_non_differentiable(*[o for o, c in zip(out, carries) if not c])
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(mask, offsets)
+        ctx.save_for_forward(mask, offsets)
+        ctx.m, ctx.spread = m, spread
         return tuple(out)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, *gout):
+        need = [g if n else None for g, n in zip(gout, ctx.needs_input_grad[5:])]
+        return None, None, None, None, None, *_MoveRows._of(ctx, 1 - ctx.spread, need)
+
+    @staticmethod
+    def jvp(ctx, _mask, _offsets, _m, _spread, _carries, *tangents):
+        return _MoveRows._of(ctx, ctx.spread, tangents)
+
+    @staticmethod
+    def _of(ctx, spread, ts):
+        """The same move, or its adjoint, of those of ts that are given."""
         mask, offsets = ctx.saved_tensors
-        res = [None] * len(gout)
-        src, dst = [], []
-        for k, g in enumerate(gout):
-            if g is None or not ctx.needs_input_grad[k + 1]:
-                continue
-            res[k] = torch.empty((mask.shape[0], *g.shape[1:]), dtype=g.dtype, device=g.device)
-            src.append(g.contiguous())
-            dst.append(res[k])
-        if src:
-            _copy_rows(mask, offsets, src, dst, 1)
-        return None, *res
+
+        def move(*t):
+            carries = tuple(map(_carries, t))
+            if not any(carries):
+                return _moved_rows(mask, offsets, ctx.m, spread, t)
+            return _MoveRows.apply(mask, offsets, ctx.m, spread, carries, *t)
+
+        return _each_given(move, ts)
 
 
 def select_rows(mask, *arrays):
     """[a[mask] for a in arrays] (a boolean mask over the first dimension): the selected rows
-    are counted once and copied in one launch.  What the kernels do not take (an empty mask,
-    rows that are no 1 to 4096 whole words, more than eight arrays) is indexed."""
+    are counted once and copied in one launch; differentiable as often as indexing is.  What the
+    kernels do not take (an empty mask, rows that are no 1 to 4096 whole words, more than eight
+    arrays) is indexed."""
     n = mask.shape[0]
     if mask.dim() == 1 and mask.dtype == torch.bool and 0 < n < 1 << 31 and 0 < len(arrays) <= 8 and mask.is_cuda and all(
             a.shape[0] == n and a.device == mask.device and a.numel() and
             a.element_size() * (a.numel() // n) % 4 == 0 and _row_words(a) <= 4096 for a in arrays):
-        return _SelectRows.apply(mask.contiguous(), *arrays)
+        mask = mask.contiguous()
+        offsets = torch.empty(lib().vx_select_blocks(n), dtype=torch.int32, device=mask.device)
+        total = torch.empty(1, dtype=torch.int64, device=mask.device)
+        call("vx_select_count", ptr(mask), n, ptr(offsets), ptr(total), stream_of(mask))
+        return _MoveRows.apply(mask, offsets, int(total.item()), 0, tuple(map(_carries, arrays)),
+                               *arrays)
     return tuple(a[mask] for a in arrays)
 
 
