@@ -69,3 +69,23 @@ def test_differentiated_twice_and_forward(dev):
         assert b.tangent is None
     for u, v in zip(*res):
         assert torch.equal(u, v)
+
+
+def test_unaligned_and_pending_values(dev):
+    """Rows of halves from an odd element, and tensors whose conjugation or sign is still to be
+    taken, as sources and as gradients."""
+    g = torch.Generator(device=dev).manual_seed(4)
+    mask = torch.rand(300, generator=g, device=dev) < 0.5
+    h = torch.randn(601, generator=g, device=dev).half()[1:].reshape(300, 2)
+    assert h.data_ptr() % 4 == 2
+    z = torch.randn(300, 2, generator=g, device=dev, dtype=torch.complex64)
+    for a in (h, z.conj(), z.conj().imag):
+        got, = select_rows(mask, a)
+        assert torch.equal(got, a[mask])
+        w = a.detach().clone().requires_grad_(True)
+        gout = a[mask]
+        if a is h:
+            gout = torch.cat([gout.new_zeros(1), gout.reshape(-1)])[1:].reshape(gout.shape)
+        ga, = torch.autograd.grad(select_rows(mask, w)[0], w, gout)
+        gb, = torch.autograd.grad(w[mask], w, gout)
+        assert torch.equal(ga, gb)

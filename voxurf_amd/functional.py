@@ -234,12 +234,21 @@ def _row_words(t):
     return t.element_size() * (t.numel() // max(t.shape[0], 1)) // 4
 
 
+def _whole_words(t):
+    """t as the row kernels read it: its own values (no pending conjugation or sign), rows on end
+    from a 4-byte boundary."""
+    if t.is_conj() or t.is_neg():
+        t = t.resolve_conj().resolve_neg()
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 4 else t
+
+
 def _moved_rows(mask, offsets, m, spread, arrays):
     """The selected rows of each array (spread 0), or its rows spread over the mask (1)."""
     n = mask.shape[0]
     out = [a.new_empty((n if spread else m, *a.shape[1:])) for a in arrays]
     if spread or m:
-        src = [a.contiguous() for a in arrays]
+        src = [_whole_words(a) for a in arrays]
         k = len(src)
         # host arrays: k sources, k destinations, k row lengths
         s, d = (ctypes.c_int64 * k)(*map(ptr, src)), (ctypes.c_int64 * k)(*map(ptr, out))
