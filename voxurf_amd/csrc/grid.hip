@@ -571,9 +571,10 @@ static bool tv_rows(const GridDesc& g, const T* param, T* grad, const T* mask, f
 }
 
 // Adjoint of k_dense_grad_fwd: gs[i] += sum_a (g_a[i - e_a] - g_a[i + e_a]) / 2 / vs over
-// interior entries.  Bound by HBM: the three gradient grids read once and gs read and written
-// take 67 us at 256^3.  A thread per element, its block's neighbours in x and y on other XCDs,
-// read them again and took 143; vectors of a plane on 16 planes in turn, as k_tv_rows, 64.
+// interior entries.  Bound by HBM: at 256^3 the three gradient grids read once and gs read and
+// written are 335 MB.  A thread per element, its block's neighbours in x and y on other XCDs,
+// read them again and took 143 us; vectors of a plane on 16 planes in turn, as k_tv_rows, 64
+// (5.2 TB/s; a large copy, half of whose bytes are writes, reaches 5.0).
 template <typename T, int V>
 __global__ void __launch_bounds__(256) k_dense_grad_bwd(const T* __restrict__ go, int X, int Y, int Z,
                                                         int depth, T vs, T* __restrict__ gs) {
