@@ -237,3 +237,27 @@ def test_alphas2weights_function(dev):
     torch.autograd.backward([w, last], [gw.to(dev), gl.to(dev)])
     rg = alpha2weight_backward(alpha.numpy(), rw, rT, rl, ris, rie, N, gw.numpy(), gl.numpy())
     close(a.grad, torch.from_numpy(rg), 1e-4)
+
+
+@pytest.mark.parametrize("form", ["plain", "rows", "planes", "expanded"])
+def test_gradients_of_grids_with_gaps(dev, form):
+    """The gradient of a grid that is a slice of a larger one, or an expanded one, is that of its
+    copy: every lookup's adjoint addresses it by strides of its own."""
+    g = torch.Generator().manual_seed(9)
+    pts = (torch.rand((300, 3), generator=g, dtype=torch.float64) * 1.8 - 0.9).to(dev)
+    mn, mx = [-1.0] * 3, [1.0] * 3
+    big = torch.randn((1, 1, 9, 10, 14), generator=g, dtype=torch.float64).to(dev)
+    view = {"plain": lambda t: t, "rows": lambda t: t[..., 2:13], "planes": lambda t: t[:, :, ::2],
+            "expanded": lambda t: t[:, :, :1].expand(1, 1, 9, 10, 14)}[form]
+    calls = [lambda q: (fn.grid_sample(q, pts, mn, mx),),
+             lambda q: fn.SdfGradSample.apply(q, pts, mn, mx, 0.15),
+             lambda q: fn.SampleSdfs.apply(q, pts, mn, mx, [0.5, 1.0], 0.15, True)]
+    for op in calls:
+        res = []
+        for copy in (False, True):
+            leaf = big.clone().requires_grad_(True)
+            q = view(leaf)
+            outs = op(q.contiguous() if copy else q)
+            sum((o * o).sum() for o in outs).backward()
+            res.append(leaf.grad)
+        assert torch.allclose(*res, rtol=1e-12, atol=1e-12)

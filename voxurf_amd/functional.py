@@ -22,8 +22,19 @@ from ._lib import call, dtype_code, lib, ptr, stream_of
 from .total_variation_cuda import grid_geom
 
 
+def _own_elements(g):
+    """g, copied where several of its entries share one element (an expanded grid)."""
+    return g.contiguous() if any(n > 1 and s == 0 for n, s in zip(g.shape, g.stride())) else g
+
+
 def _zeros_like_grid(g):
-    return torch.zeros_like(g, memory_format=torch.preserve_format)
+    """Zeros with g's strides (the kernels address the gradient by the grid's), also where g has
+    gaps between its rows, which zeros_like closes."""
+    z = torch.zeros_like(g, memory_format=torch.preserve_format)
+    if z.stride() == g.stride():
+        return z
+    span = 1 + sum((n - 1) * s for n, s in zip(g.shape, g.stride()))
+    return g.new_zeros(span).as_strided(g.shape, g.stride())
 
 
 def _dev_vec(v, like):
@@ -37,7 +48,7 @@ class GridSample(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, grid, xyz, xyz_min, xyz_max):
-        xyz = xyz.contiguous()
+        grid, xyz = _own_elements(grid), xyz.contiguous()
         mn, mx = _dev_vec(xyz_min, grid), _dev_vec(xyz_max, grid)
         geom = grid_geom(grid)
         out = torch.empty((xyz.shape[0], grid.shape[1]), dtype=grid.dtype, device=grid.device)
@@ -69,7 +80,7 @@ class SdfGradSample(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, grid, xyz, xyz_min, xyz_max, voxel_size):
-        xyz = xyz.contiguous()
+        grid, xyz = _own_elements(grid), xyz.contiguous()
         mn, mx = _dev_vec(xyz_min, grid), _dev_vec(xyz_max, grid)
         geom = grid_geom(grid)
         n = xyz.shape[0]
@@ -103,7 +114,7 @@ class SampleSdfs(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, grid, xyz, xyz_min, xyz_max, displace, voxel_size, use_grad_norm):
-        xyz = xyz.contiguous()
+        grid, xyz = _own_elements(grid), xyz.contiguous()
         mn, mx = _dev_vec(xyz_min, grid), _dev_vec(xyz_max, grid)
         disp = _dev_vec(list(displace), grid)
         nd = disp.numel()
