@@ -96,11 +96,12 @@ def _prefilter_args(mask_cache, xyz_min, xyz_max, near, stepdist):
 # need the bits (a pass over the cache's grid: 85 us for 256^3) and a thread a ray, whose chain
 # of steps is as long for one ray as for many; a wavefront a ray that looks every sample up is
 # through after a few chunks of 64.  Whole calls in us, wavefront / bits, for a shell in a 100^3
-# cache at steps of a voxel: 8192 rays 21 / 58, 32768 42 / 61, 65536 75 / 61; views of 200^2
-# pixels 127 / 342, 400^2 292 / 419, 460^2 364 / 447, 512^2 452 / 346 (256^3: 835 / 741 at
-# 460^2; an empty cache sooner: 218 / 147 at 300^2, but no step in it is looked up).
+# cache at steps of half a voxel of 96^3: 8192 rays 21 / 58, 32768 42 / 61, 65536 75 / 61; views
+# of 200 x 266 pixels 186 / 417, 300 x 400 285 / 339, 380 x 506 393 / 363, 600 x 800 832 / 351
+# (of 255^3: 265 / 600, 459 / 534, 672 / 599, 1501 / 609; an empty cache sooner: 218 / 147 for
+# 300 x 300).
 OCC_RAYS = 1 << 15
-OCC_PIXELS = 200000
+OCC_PIXELS = 160000
 
 
 def _occupancy(mask_cache, mc):
