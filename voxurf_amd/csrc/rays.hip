@@ -393,8 +393,9 @@ __global__ void __launch_bounds__(256) k_hit_rays(FusedGeom G, Occupancy oc,
 // Measured on 1.92 M rays of a 1200 x 1600 view at half-voxel steps of 256^3: a wavefront per
 // ray that looked every sample up (64 at a time, eight loads, exp and log1p each) 5,480 us;
 // a thread per ray jumping over clear bricks and blocks 1,200 us (410 M vector instructions,
-// 140 jumps a wave); with the tiles' stretches 614 us (205 M).
-__global__ void __launch_bounds__(256) k_hit_camera(FusedGeom G, Occupancy oc, Camera c,
+// 140 jumps a wave); with the tiles' stretches 614 us (205 M).  Five waves a SIMD: with the
+// registers for four the view took 30 us longer.
+__global__ void __launch_bounds__(256, 5) k_hit_camera(FusedGeom G, Occupancy oc, Camera c,
                                                     int64_t* __restrict__ flag) {
   const int words = (oc.bx * oc.by * oc.bz + 31) >> 5;
   const uint32_t* bits = occ_to_lds(oc.bits, words, 0);

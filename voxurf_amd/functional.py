@@ -24,7 +24,9 @@ from .total_variation_cuda import grid_geom
 
 def _own_elements(g):
     """g, copied where several of its entries share one element (an expanded grid)."""
-    return g.contiguous() if any(n > 1 and s == 0 for n, s in zip(g.shape, g.stride())) else g
+    strides = g.stride()
+    return g.contiguous() if 0 in strides and any(
+        n > 1 and s == 0 for n, s in zip(g.shape, strides)) else g
 
 
 def _zeros_like_grid(g):
