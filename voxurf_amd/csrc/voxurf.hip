@@ -60,8 +60,8 @@ __device__ __forceinline__ void hier_lane(const FusedGeom& G, const VoxurfRowDes
 // 6 nd displaced samples of a row (minus and plus in neighbouring lanes), the sines and
 // cosines (once for both rows), four channels of k0.  A wavefront per ray with sixteen lanes a
 // row before, twelve of them taking two samples in turn and each working out its columns'
-// embeddings with runtime divisions, was bound by those instructions: 491 us for 29,000 rows
-// of an 8192-ray chunk, 50 so.  XK's logit columns are left zero (vx_voxurf_logit_cols
+// embeddings with runtime divisions, was bound by those instructions: 491 us for 96,000 rows
+// of an 8192-ray chunk, 51 so.  XK's logit columns are left zero (vx_voxurf_logit_cols
 // fills them after rgbnet's forward).
 constexpr int kVxRowTile = 32;
 
