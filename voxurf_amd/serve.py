@@ -173,7 +173,7 @@ class ResidentScene:
         (x_i = -1 + 2 i / (res - 1)): points [tile^3, 3] -> (sdf [P], normal [P, 3])."""
         i0, j0, k0 = tile_origin  # three of them: the kernel's call reads that many
         origin = np.array([float(i0), float(j0), float(k0)], dtype=np.float32)
-        tile = math.ceil(tile)    # as many points as arange(tile) has
+        tile = math.ceil(float(tile))    # as many points as arange(tile) has
         if tile < 0:
             raise ValueError("sdf_query: negative tile")
         n = tile ** 3
